@@ -155,13 +155,60 @@ void exchange_blocks(hipStream_t s, int W, int n, int mg, int MC, int m0, int mc
                      const cplx<TT>* T, z64* exx_part, int ng_total, int g0, z64* Kl);
 void energy_finish(hipStream_t s, int W, int M, int nchunk, const z64* exx_part, const z64* Kl,
                    double cx, double cj, int addEXX, int addEJ, z64* E);
-// Fused FP32 exchange of a real half-rotated tensor (exchange.hip): T^m = G_w L^m^T formed and
-// reduced on chip.  G [W][ns][N] complex64, L [M][ns][N] real; part [W][nparts] exchange
-// partials (nparts = exx_fused_parts(M)), Kl[w][m] += tr T^m (Kl may be null).
-bool exx_fused_supported(int ns, int N, int M);
-int exx_fused_vpw();
+// Fused FP32 exchange of a real half-rotated tensor (exchange.hip): T^m = G_w L^m^T formed on the
+// bfloat16 matrix cores (split3.hpp) and reduced on chip.  G packed by s3::pack_exx_G, L by
+// s3::pack_exx_L; part [W][nparts] exchange partials (nparts = exx_fused_parts(M)),
+// Kl[w][m] += tr T^m (Kl may be null).
 int exx_fused_parts(int M);
-void exchange_fused(hipStream_t s, int W, int ns, int N, int M, const c32* G, const float* L,
+void exchange_fused(hipStream_t s, int W, int ns, int N, int M, const void* G, const void* L,
                     z64* part, int nparts, z64* Kl);
+
+// ---- split3.hip: FP32 products on the bfloat16 matrix cores ------------------------------------
+namespace s3 {
+constexpr long kBlock = 3072;  // bytes of a packed block of 16 rows x 32 k values
+inline long k_groups(long K) { return (K + 31) / 32; }
+inline long row_blocks(long rows) { return (rows + 15) / 16; }
+// bytes of a packed real operand of `rows` rows, and of a complex one
+inline size_t bytes_real(long rows, long K) {
+  return (size_t)(row_blocks(rows) * k_groups(K) * kBlock);
+}
+inline size_t bytes_cplx(long rows, long K) { return 2 * bytes_real(rows, K); }
+// The packed operands are read with 32-bit offsets.
+inline bool fits(long rows, long K, bool cplx_rows) {
+  return (cplx_rows ? bytes_cplx(rows, K) : bytes_real(rows, K)) < (size_t)0xFFFF0000u;
+}
+// Pack a complex operand [rows][ld] (values rounded to FP32), or the rows of a real one; *bad is
+// set when a value of a real operand is not finite.  pack_pairs: row n is the orbital pair
+// pairs[n] = i << 16 | k of an [N * N][K] tensor.
+void pack_cplx(hipStream_t s, int rows, int K, const c32* X, long ld, void* out);
+void pack_cplx(hipStream_t s, int rows, int K, const z64* X, long ld, void* out);
+void pack_rows(hipStream_t s, int rows, int K, const float* X, long ld, void* out, int* bad);
+void pack_pairs(hipStream_t s, int rows, int K, const float* X, int N, const uint32_t* pairs,
+                void* out, int* bad);
+// The operands of the exchange kernel (n <= 40): tiles of two walkers (G [W][n][N], real parts then
+// imaginary parts) and of two Cholesky vectors (L [M][n][N]), each item's n rows padded to 8 nb,
+// so a tile is nb 16-row blocks; an odd last item is padded with zeros.
+inline int exx_nb(int n) { return (n + 7) / 8; }
+inline size_t bytes_exx_G(long W, int n, long N) {
+  return (size_t)((W + 1) / 2 * 2 * exx_nb(n) * k_groups(N) * kBlock);
+}
+inline size_t bytes_exx_L(long M, int n, long N) {
+  return (size_t)((M + 1) / 2 * exx_nb(n) * k_groups(N) * kBlock);
+}
+void pack_exx_G(hipStream_t s, int W, int n, int N, const z64* G, void* out);
+void pack_exx_L(hipStream_t s, int M, int n, int N, const float* L, void* out, int* bad);
+// V[w][i][k] = V[w][k][i] = alpha sum_m A[w][m] B[p][m] over the np pairs p = (i, k), from the last m
+// to the first
+void vhs_pairs(hipStream_t s, int W, int np, int K, const void* A, const void* B,
+               const uint32_t* pairs, int N, float alpha, c32* V);
+// v[w][m] (+)= alpha sum_k A[w][k] B[m][k], K cut into p.ksplit slices (ws [ksplit][W][M] when
+// more than one)
+struct Plan {
+  int tile, ksplit, kchunk;
+};
+Plan plan(int M, int N, int KG, bool split_k);
+void vbias(hipStream_t s, int W, int M, int K, const void* A, const void* B, const Plan& p,
+           float alpha, bool accumulate, z64* v, c32* ws);
+}  // namespace s3
 
 }  // namespace afq

@@ -105,7 +105,13 @@ CholeskyOps::CholeskyOps(Context& c, int walker_type, int N, int nup, int ndown,
     Lnak_r_ = own.Lnak_r;
     Lnak_r32_ = own.Lnak_r32;
     Lnak32_ = own.Lnak32;
+    Lnak_s3_ = own.Lnak_s3;
+    s3_off_[0] = own.s3_off[0];
+    s3_off_[1] = own.s3_off[1];
+    Lexx_s3_[0] = own.Lexx_s3[0];
+    Lexx_s3_[1] = own.Lexx_s3[1];
     real_trial_ = own.real;
+    build_pairs();
     AFQ_HIP(hipStreamSynchronize(s));
   } catch (...) {
     free_all();
@@ -169,6 +175,7 @@ void CholeskyOps::half_rotate_into(const z64* PsiT, Rotated& r) const {
       if (r.real) {
         r.Lnak_r32 = dalloc<float>((size_t)M * nel_ * N);
         real_part_f32(s, (long)M * nel_ * N, r.Lnak, r.Lnak_r32);
+        build_split(r);
       } else {
         r.Lnak32 = dalloc<c32>((size_t)M * nel_ * N);
         cast_z64_c32(s, (long)M * nel_ * N, r.Lnak, r.Lnak32);
@@ -177,6 +184,76 @@ void CholeskyOps::half_rotate_into(const z64* PsiT, Rotated& r) const {
   } catch (...) {
     release(r);
     throw;
+  }
+}
+
+// The FP32 half-rotated tensor split into bfloat16 pieces (split3.hpp): per spin block packed by
+// rows (m) over (a, k) for vbias and by tiles of two vectors for the exchange.  A tensor that is not
+// finite or beyond the packed operands' 32-bit offsets keeps the FP32 products.
+void CholeskyOps::build_split(Rotated& r) const {
+  hipStream_t s = ctx_.stream();
+  const int N = N_, M = M_, ns[2] = {nup_, ndown_};
+  int* bad = scratch_as<int>(ctx_, "setup_bad", 1);
+  AFQ_HIP(hipMemsetAsync(bad, 0, sizeof(int), s));
+  r.s3_off[1] = s3::bytes_real(M, (long)nup_ * N);
+  if (s3::fits(M, (long)std::max(nup_, ndown_) * N, false))
+    r.Lnak_s3 = dalloc<char>(r.s3_off[1] + s3::bytes_real(M, (long)ndown_ * N));
+  for (int sp = 0; sp < 2; ++sp) {
+    if (ns[sp] == 0) continue;
+    const float* L = r.Lnak_r32 + (sp == 0 ? 0 : (size_t)M * nup_ * N);
+    if (r.Lnak_s3)
+      s3::pack_rows(s, M, ns[sp] * N, L, (long)ns[sp] * N, r.Lnak_s3 + r.s3_off[sp], bad);
+    const size_t eb = s3::bytes_exx_L(M, ns[sp], N);
+    if (std::max(nup_, ndown_) <= 40 && eb < (size_t)0xFFFF0000u) {
+      r.Lexx_s3[sp] = dalloc<char>(eb);
+      s3::pack_exx_L(s, M, ns[sp], N, L, r.Lexx_s3[sp], bad);
+    }
+  }
+  int hbad = 0;
+  AFQ_HIP(hipMemcpyAsync(&hbad, bad, sizeof(int), hipMemcpyDeviceToHost, s));
+  AFQ_HIP(hipStreamSynchronize(s));
+  if (!hbad) return;
+  for (char** p : {&r.Lnak_s3, &r.Lexx_s3[0], &r.Lexx_s3[1]}) {
+    (void)hipFree(*p);
+    *p = nullptr;
+  }
+}
+
+// The orbital pairs (i <= k) that vHS computes and the packed rows L[i][k] (mixed precision).  The
+// pairs run through the full 8 x 8 blocks above the diagonal, block by block (so that both mirrored
+// stores of eight neighbouring columns fill whole 64-byte lines), then through the diagonal
+// blocks' triangles and the ragged last block column.
+void CholeskyOps::build_pairs() {
+  if (prec_ != kMixed || !sym_L_ || N_ > 0xFFFF) return;
+  const long np = (long)N_ * (N_ + 1) / 2;
+  if (!s3::fits(np, M_, false)) return;
+  hipStream_t s = ctx_.stream();
+  std::vector<uint32_t> h;
+  h.reserve(np);
+  const int nb = ceil_div(N_, 8);
+  for (int pass = 0; pass < 2; ++pass)
+    for (int bi = 0; bi < nb; ++bi)
+      for (int bk = bi; bk < nb; ++bk) {
+        if ((bk > bi && 8 * bk + 8 <= N_) != (pass == 0)) continue;
+        for (int i = 8 * bi; i < std::min(8 * bi + 8, N_); ++i)
+          for (int k = std::max(i, 8 * bk); k < std::min(8 * bk + 8, N_); ++k)
+            h.push_back((uint32_t)i << 16 | (uint32_t)k);
+      }
+  pairs_ = dalloc<uint32_t>(np);
+  AFQ_HIP(hipMemcpyAsync(pairs_, h.data(), sizeof(uint32_t) * np, hipMemcpyHostToDevice, s));
+  const size_t bytes = s3::bytes_real(np, M_);
+  Lpair_s3_ = dalloc<char>(nl_ * bytes);
+  int* bad = scratch_as<int>(ctx_, "setup_bad", 1);
+  AFQ_HIP(hipMemsetAsync(bad, 0, sizeof(int), s));
+  for (int l = 0; l < nl_; ++l)
+    s3::pack_pairs(s, (int)np, M_, Likn32_ + (size_t)l * N_ * N_ * M_, N_, pairs_,
+                   Lpair_s3_ + l * bytes, bad);
+  int hbad = 0;
+  AFQ_HIP(hipMemcpyAsync(&hbad, bad, sizeof(int), hipMemcpyDeviceToHost, s));
+  AFQ_HIP(hipStreamSynchronize(s));
+  if (hbad) {  // not finite: the FP32 products keep their infinities
+    (void)hipFree(Lpair_s3_);
+    Lpair_s3_ = nullptr;
   }
 }
 
@@ -190,14 +267,16 @@ Rotated CholeskyOps::rotate(const z64* PsiT) const {
 void CholeskyOps::release(Rotated& r) const {
   (void)hipStreamSynchronize(ctx_.stream());
   for (void* p : {(void*)r.PsiT, (void*)r.Lnak, (void*)r.haj, (void*)r.Lnak_r, (void*)r.Lnak_r32,
-                  (void*)r.Lnak32})
+                  (void*)r.Lnak32, (void*)r.Lnak_s3, (void*)r.Lexx_s3[0], (void*)r.Lexx_s3[1]})
     if (p) (void)hipFree(p);
   r = Rotated{};
 }
 
 void CholeskyOps::free_all() {
   for (void* p : {(void*)PsiT_, (void*)Likn_, (void*)Likn32_, (void*)h1_, (void*)vexx_,
-                  (void*)Lnak_, (void*)Lnak_r_, (void*)Lnak_r32_, (void*)Lnak32_, (void*)haj_})
+                  (void*)Lnak_, (void*)Lnak_r_, (void*)Lnak_r32_, (void*)Lnak32_, (void*)haj_,
+                  (void*)Lpair_s3_, (void*)pairs_, (void*)Lnak_s3_, (void*)Lexx_s3_[0],
+                  (void*)Lexx_s3_[1]})
     if (p) (void)hipFree(p);
   PsiT_ = nullptr;
   Likn_ = nullptr;
@@ -208,6 +287,8 @@ void CholeskyOps::free_all() {
   Lnak_r32_ = nullptr;
   Lnak32_ = nullptr;
   haj_ = nullptr;
+  Lpair_s3_ = Lnak_s3_ = Lexx_s3_[0] = Lexx_s3_[1] = nullptr;
+  pairs_ = nullptr;
 }
 
 CholeskyOps::~CholeskyOps() {
@@ -217,6 +298,10 @@ CholeskyOps::~CholeskyOps() {
 
 void CholeskyOps::vbias(const z64* G, int W, double dt, z64* v, Precision prec) const {
   if (W == 0) return;
+  if (prec != kFP64) {
+    vbias_f32(G, W, dt, v);
+    return;
+  }
   hipStream_t s = ctx_.stream();
   const double a = std::sqrt(dt) * (walker_type_ == kClosed ? 2.0 : 1.0);
   const int nel_ = nel();
@@ -231,7 +316,7 @@ void CholeskyOps::vbias(const z64* G, int W, double dt, z64* v, Precision prec) 
     size_t goff = sp == 0 ? 0 : (size_t)nup_ * N_;
     size_t loff = sp == 0 ? 0 : (size_t)M_ * nup_ * N_;
     const long K = (long)ns * N_;
-    if (prec == kFP64) {
+    {
       // A(w, (a,k)) = G[w][off + a][k]: rows of length nel*N, K = ns*N contiguous
       Opnd<double, true, true> A{&(G + goff)->re, (long)nel_ * N_, 0};
       EpiStore<double, double> e{v, M_, 0, a, 0, acc};
@@ -250,17 +335,6 @@ void CholeskyOps::vbias(const z64* G, int W, double dt, z64* v, Precision prec) 
       } else {
         Opnd<double, true, true> B{&(Lnak_ + loff)->re, K, 0};
         gemm_large_splitk<double>(ctx_, "vbias_c", W, M_, (int)K, A, B, e, acc == 0);
-      }
-    } else {
-      AFQ_CHECK(prec_ == kMixed, kErrState, "FP32 tensors were not built (precision FP64)");
-      Opnd<double, true, true> A{&(G + goff)->re, (long)nel_ * N_, 0};
-      EpiStore<float, double> e{v, M_, 0, (float)a, 0.f, acc};
-      if (real_trial_) {
-        Opnd<float, false, true> B{Lnak_r32_ + loff, K, 0};
-        gemm_large_splitk<float>(ctx_, "vbias_r", W, M_, (int)K, A, B, e, acc == 0);
-      } else {
-        Opnd<float, true, true> B{&(Lnak32_ + loff)->re, K, 0};
-        gemm_large_splitk<float>(ctx_, "vbias_c", W, M_, (int)K, A, B, e, acc == 0);
       }
     }
   }
@@ -300,13 +374,14 @@ void CholeskyOps::vHS(const void* X, int W, double dt, void* V, Precision prec) 
         AFQ_CHECK(prec_ == kMixed, kErrState, "FP32 tensors were not built (precision FP64)");
         gemm::EpiStoreSym<float, float> e{reinterpret_cast<c32*>(Vl), NN, 0, (float)a, 0.f, N_, nb};
         const c32* X32 = reinterpret_cast<const c32*>(X);
-        if (crg_path() && crg::crg_supported<float>(X32, M_, W, Likn32_ + loff, M_, NN) &&
-            crg::crg_fills(W, npairs, 4, 7)) {
-          // register-tiled: 64 walkers x 112 pairs per wavefront, k groups from the last
-          // Cholesky vector to the first
-          crg::launch_crgemm<float, 4, 7, true>(s, W, npairs, M_, X32, M_, Likn32_ + loff,
-                                                crg::RowsSymPairs{M_, N_, nb}, 1,
-                                                ceil_div(M_, 16) * 16, e, nullptr);
+        if (Lpair_s3_ && crg_path() && s3::fits(W, M_, true)) {
+          // on the bfloat16 matrix cores over the N(N+1)/2 distinct pairs, k groups from the
+          // last Cholesky vector to the first
+          const int np = N_ * (N_ + 1) / 2;
+          char* A = scratch_as<char>(ctx_, "s3_A", s3::bytes_cplx(W, M_));
+          if (l == 0) s3::pack_cplx(s, W, M_, X32, M_, A);
+          s3::vhs_pairs(s, W, np, M_, A, Lpair_s3_ + l * s3::bytes_real(np, M_), pairs_, N_,
+                        (float)a, reinterpret_cast<c32*>(Vl));
         } else {
           gemm::RevK<Opnd<float, true, true>> A({reinterpret_cast<const float*>(X), M_, 0}, M_);
           gemm::RevK<gemm::OpndSymPairs<float>> B({Likn32_ + loff, M_, 0, N_, nb}, M_);
@@ -332,6 +407,11 @@ void CholeskyOps::vHS(const void* X, int W, double dt, void* V, Precision prec) 
 }
 
 void CholeskyOps::vbias32(const c32* G, int W, double dt, z64* v) const {
+  vbias_f32(G, W, dt, v);
+}
+
+template <typename TG>
+void CholeskyOps::vbias_f32(const cplx<TG>* G, int W, double dt, z64* v) const {
   if (W == 0) return;
   AFQ_CHECK(prec_ == kMixed, kErrState, "FP32 tensors were not built (precision FP64)");
   hipStream_t s = ctx_.stream();
@@ -347,24 +427,26 @@ void CholeskyOps::vbias32(const c32* G, int W, double dt, z64* v) const {
     size_t goff = sp == 0 ? 0 : (size_t)nup_ * N_;
     size_t loff = sp == 0 ? 0 : (size_t)M_ * nup_ * N_;
     const long K = (long)ns * N_;
-    Opnd<float, true, true> A{&(G + goff)->re, (long)nel_ * N_, 0};
     EpiStore<float, double> e{v, M_, 0, a, 0.f, acc};
-    int ks = 0, kc = 0;
-    if (real_trial_ && crg_path() &&
-        crg::crg_supported<float>(G + goff, (long)nel_ * N_, W, Lnak_r32_ + loff, K, M_))
-      crg::crg_split(W, M_, (int)K, 4, 7, ks, kc);
-    if (ks > 0 && crg::crg_fills(W, M_, 4, 7, ks)) {
-      // register-tiled, K cut into slices so that the 64 x 112 tiles fill the machine
-      cplx<float>* ws =
-          ks > 1 ? scratch_as<cplx<float>>(ctx_, "crg_ws32", (size_t)ks * W * M_) : nullptr;
-      crg::launch_crgemm<float, 4, 7, false>(s, W, M_, (int)K, G + goff, (long)nel_ * N_,
-                                             Lnak_r32_ + loff, crg::RowsPlain{K}, ks, kc, e, ws);
-    } else if (real_trial_) {
+    if (Lnak_s3_ && crg_path() && s3::fits(W, K, true)) {
+      // on the bfloat16 matrix cores, K cut into slices so that the tiles fill the machine
+      char* A = scratch_as<char>(ctx_, "s3_A", s3::bytes_cplx(W, K));
+      s3::pack_cplx(s, W, (int)K, G + goff, (long)nel_ * N_, A);
+      const s3::Plan p = s3::plan(W, M_, (int)s3::k_groups(K), true);
+      c32* ws = p.ksplit > 1 ? scratch_as<c32>(ctx_, "s3_ws", (size_t)p.ksplit * W * M_) : nullptr;
+      s3::vbias(s, W, M_, (int)K, A, Lnak_s3_ + s3_off_[sp], p, a, acc != 0, v, ws);
+      continue;
+    }
+    constexpr bool g32 = sizeof(TG) == 4;
+    Opnd<TG, true, true> A{&(G + goff)->re, (long)nel_ * N_, 0};
+    if (real_trial_) {
       Opnd<float, false, true> B{Lnak_r32_ + loff, K, 0};
-      gemm_large_splitk<float>(ctx_, "vbias32_r", W, M_, (int)K, A, B, e, acc == 0);
+      gemm_large_splitk<float>(ctx_, g32 ? "vbias32_r" : "vbias_r", W, M_, (int)K, A, B, e,
+                               acc == 0);
     } else {
       Opnd<float, true, true> B{&(Lnak32_ + loff)->re, K, 0};
-      gemm_large_splitk<float>(ctx_, "vbias32_c", W, M_, (int)K, A, B, e, acc == 0);
+      gemm_large_splitk<float>(ctx_, g32 ? "vbias32_c" : "vbias_c", W, M_, (int)K, A, B, e,
+                               acc == 0);
     }
   }
 }
@@ -396,21 +478,21 @@ void CholeskyOps::vbias_full(const z64* G, int W, double dt, z64* v, Precision p
 // Kl is given, Kl[w][m] += tr T^m.  Gblk [W][ns][N] contiguous.  The Cholesky vectors are taken
 // in chunks whose T [W][ns][MC][ns] fits 1 GiB (max_memory_MB of energy_impl,
 // Real3IndexFactorization.hpp:511-587), sized for the larger spin block so both share the buffer.
-// The register-tiled products of crgemm.hpp (FP32 and FP64) for vHS and vbias; AFQ_CRGEMM=0
+// The register-tiled products of vHS and vbias (FP64: crgemm.hpp, FP32: split3.hpp); AFQ_CRGEMM=0
 // selects the LDS-staged GEMM engine instead.
 bool CholeskyOps::crg_path() {
   const char* e = std::getenv("AFQ_CRGEMM");
   return !(e && e[0] == '0');
 }
 
-bool CholeskyOps::exchange_fused_path(Precision prec, bool real) const {
+bool CholeskyOps::exchange_fused_path(Precision prec, const Rotated& t) const {
   const char* e = std::getenv("AFQ_EXX_FUSED");  // "0": the GEMM + reduction path
-  return prec != kFP64 && real && exx_fused_supported(std::max(nup_, ndown_), N_, M_) &&
+  return prec != kFP64 && (nup_ == 0 || t.Lexx_s3[0]) && (ndown_ == 0 || t.Lexx_s3[1]) &&
          !(e && e[0] == '0');
 }
 
-int CholeskyOps::exchange_parts(Precision prec, bool real) const {
-  return exchange_fused_path(prec, real)
+int CholeskyOps::exchange_parts(Precision prec, const Rotated& t) const {
+  return exchange_fused_path(prec, t)
              ? exx_fused_parts(M_)
              : ceil_div(M_, exchange_group(std::max(std::max(nup_, ndown_), 1)));
 }
@@ -420,12 +502,18 @@ void CholeskyOps::exchange_spin(int sp, const z64* Gblk, int W, z64* part, z64* 
   hipStream_t s = ctx_.stream();
   const int ns = sp == 0 ? nup_ : ndown_;
   const int nmax = std::max(nup_, ndown_);
-  if (exchange_fused_path(prec, t.real)) {
-    AFQ_CHECK(prec_ == kMixed, kErrState, "FP32 tensors were not built (precision FP64)");
-    c32* G32 = scratch_as<c32>(ctx_, "en_G32", (size_t)W * ns * N_);
-    cast_z64_c32(s, (long)W * ns * N_, Gblk, G32);
-    const size_t loff = sp == 0 ? 0 : (size_t)M_ * nup_ * N_;
-    exchange_fused(s, W, ns, N_, M_, G32, t.Lnak_r32 + loff, part, exx_fused_parts(M_), Kl);
+  if (exchange_fused_path(prec, t)) {
+    // walkers in runs (of even length) whose packed G stays below 2 GiB
+    const int nparts = exx_fused_parts(M_);
+    const size_t per2 = s3::bytes_exx_G(2, ns, N_);
+    const int run = 2 * (int)std::max<size_t>(1, (size_t)0x7FFF0000u / per2);
+    char* Gp = scratch_as<char>(ctx_, "s3_A", s3::bytes_exx_G(std::min(W, run), ns, N_));
+    for (int w = 0; w < W; w += run) {
+      const int wc = std::min(run, W - w);
+      s3::pack_exx_G(s, wc, ns, N_, Gblk + (size_t)w * ns * N_, Gp);
+      exchange_fused(s, wc, ns, N_, M_, Gp, t.Lexx_s3[sp], part + (size_t)w * nparts, nparts,
+                     Kl ? Kl + (size_t)w * M_ : nullptr);
+    }
     return;
   }
   const bool t32 = prec != kFP64;
@@ -495,7 +583,7 @@ void CholeskyOps::energy(const z64* G, int W, z64* E, bool addH1, bool addEJ, bo
   z64* Kl = scratch_as<z64>(ctx_, "en_Kl", (size_t)W * M_);
   fill_z64(s, (long)W * M_, {0, 0}, Kl);
   const int nspin = walker_type_ == kCollinear ? 2 : 1;
-  const int ng_total = exchange_parts(prec, t.real);
+  const int ng_total = exchange_parts(prec, t);
   z64* part = scratch_as<z64>(ctx_, "en_part", (size_t)W * ng_total * nspin);
   for (int sp = 0; sp < nspin; ++sp) {
     int ns = sp == 0 ? nup_ : ndown_;
@@ -538,7 +626,7 @@ void CholeskyOps::energy_spin(int spin, const z64* G, int W, z64* E, z64* EJn, b
   if (addH1)
     dot_rows(s, W, (long)ns * N_, G, haj_ + (spin == 0 ? 0 : (size_t)nup_ * N_), c, 0.0, 0.0, E, 3);
   if (!addEXX) return;
-  const int ng_total = exchange_parts(prec, real_trial_);
+  const int ng_total = exchange_parts(prec, self());
   z64* part = scratch_as<z64>(ctx_, "ens_part", (size_t)W * ng_total);
   exchange_spin(spin, G, W, part, addEJ ? EJn : nullptr, prec, self());
   // E[w][1] = -1/2 c sum exx;  E[w][2] = 1/2 sum_m EJn^2 (:206-207)

@@ -1,12 +1,11 @@
-// Register-tiled product of a complex operand and a real operand, both K-contiguous, in FP32 or
-// FP64:
+// Register-tiled FP64 product of a complex operand and a real operand, both K-contiguous:
 //
 //   C(m, n) = sum_k A(m, k) * B(n, k)      A complex [M][lda], B real [N rows][K]
 //
 // the shape of vHS (A = the fields X [W][M], B = the Cholesky vectors' symmetric pairs) and of
 // vbias (A = the walkers' G, B = the half-rotated Cholesky vectors).  Each wavefront owns a
-// 16 RB x 16 CB tile of C in MFMA accumulators (v_mfma_f32_16x16x4f32 or v_mfma_f64_16x16x4f64,
-// 2 MFMAs per block: re(A) B and im(A) B) and streams its operands from memory straight into
+// 16 RB x 16 CB tile of C in MFMA accumulators (v_mfma_f64_16x16x4f64, 2 MFMAs per block: re(A) B
+// and im(A) B) and streams its operands from memory straight into
 // MFMA fragments: lane (fr, fk) of k group g feeds MFMA step j with k = 16 g + 4 fk + j, four
 // consecutive k values per lane, so the fragments are whole 16-byte words.  There is no LDS and
 // no barrier: per k group a wavefront issues its fragment loads and 8 RB CB MFMAs, the next
@@ -17,7 +16,7 @@
 // valid row and are never stored.  Operands are addressed by 32-bit byte offsets from uniform
 // bases (crg_supported checks the sizes).  The ragged last k group is taken first; with REVK the
 // full groups then run from last to first, so an accumulation over Cholesky vectors ordered by
-// decreasing norm adds the small terms first.  Split-K slices write FP32 partials that kreduce_splitk sums in slice
+// decreasing norm adds the small terms first.  Split-K slices write partials that kreduce_splitk sums in slice
 // order; every result depends on the shape only.
 #pragma once
 
@@ -67,58 +66,26 @@ __device__ inline void load(Frag<T, RB, CB>& f, const char* ab, const char* bb,
                             const Ofs<RB, CB>& o, int rem) {
 #pragma unroll
   for (int i = 0; i < RB; ++i) {
-    if constexpr (sizeof(T) == 4) {
-      const float4 z = {0.f, 0.f, 0.f, 0.f};
-      float4 x = z, y = z;
-      if (FULL || rem >= 4) {
-        x = *reinterpret_cast<const float4*>(ab + o.a[i]);
-        y = *reinterpret_cast<const float4*>(ab + o.a[i] + 16);
-      } else {
-        float2 t[4] = {{0.f, 0.f}, {0.f, 0.f}, {0.f, 0.f}, {0.f, 0.f}};
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          if (rem > j) t[j] = *reinterpret_cast<const float2*>(ab + o.a[i] + 8 * j);
-        x = float4{t[0].x, t[0].y, t[1].x, t[1].y};
-        y = float4{t[2].x, t[2].y, t[3].x, t[3].y};
-      }
-      f.ar[i][0] = x.x; f.ai[i][0] = x.y; f.ar[i][1] = x.z; f.ai[i][1] = x.w;
-      f.ar[i][2] = y.x; f.ai[i][2] = y.y; f.ar[i][3] = y.z; f.ai[i][3] = y.w;
-    } else {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        double2 v = {0.0, 0.0};
-        if (FULL || rem > j) v = *reinterpret_cast<const double2*>(ab + o.a[i] + 16 * j);
-        f.ar[i][j] = v.x;
-        f.ai[i][j] = v.y;
-      }
+    for (int j = 0; j < 4; ++j) {
+      double2 v = {0.0, 0.0};
+      if (FULL || rem > j) v = *reinterpret_cast<const double2*>(ab + o.a[i] + 16 * j);
+      f.ar[i][j] = v.x;
+      f.ai[i][j] = v.y;
     }
   }
 #pragma unroll
   for (int jb = 0; jb < CB; ++jb) {
-    if constexpr (sizeof(T) == 4) {
-      float4 x = {0.f, 0.f, 0.f, 0.f};
-      if (FULL || rem >= 4) {
-        x = *reinterpret_cast<const float4*>(bb + o.b[jb]);
-      } else {
-        float t[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          if (rem > j) t[j] = *reinterpret_cast<const float*>(bb + o.b[jb] + 4 * j);
-        x = float4{t[0], t[1], t[2], t[3]};
-      }
-      f.b[jb][0] = x.x; f.b[jb][1] = x.y; f.b[jb][2] = x.z; f.b[jb][3] = x.w;
+    double2 x = {0.0, 0.0}, y = {0.0, 0.0};
+    if (FULL || rem >= 4) {
+      x = *reinterpret_cast<const double2*>(bb + o.b[jb]);
+      y = *reinterpret_cast<const double2*>(bb + o.b[jb] + 16);
     } else {
-      double2 x = {0.0, 0.0}, y = {0.0, 0.0};
-      if (FULL || rem >= 4) {
-        x = *reinterpret_cast<const double2*>(bb + o.b[jb]);
-        y = *reinterpret_cast<const double2*>(bb + o.b[jb] + 16);
-      } else {
-        if (rem > 0) x.x = *reinterpret_cast<const double*>(bb + o.b[jb]);
-        if (rem > 1) x.y = *reinterpret_cast<const double*>(bb + o.b[jb] + 8);
-        if (rem > 2) y.x = *reinterpret_cast<const double*>(bb + o.b[jb] + 16);
-      }
-      f.b[jb][0] = x.x; f.b[jb][1] = x.y; f.b[jb][2] = y.x; f.b[jb][3] = y.y;
+      if (rem > 0) x.x = *reinterpret_cast<const double*>(bb + o.b[jb]);
+      if (rem > 1) x.y = *reinterpret_cast<const double*>(bb + o.b[jb] + 8);
+      if (rem > 2) y.x = *reinterpret_cast<const double*>(bb + o.b[jb] + 16);
     }
+    f.b[jb][0] = x.x; f.b[jb][1] = x.y; f.b[jb][2] = y.x; f.b[jb][3] = y.y;
   }
 }
 
@@ -217,8 +184,7 @@ __global__ void __launch_bounds__(64 * kWaves)
 }
 
 // The kernel's requirements: 32-bit byte offsets reach every row of A and B, and the fragment
-// loads are 16-byte aligned (the bases 16-byte aligned, A rows of an even number of complex
-// elements in FP32, B rows of a multiple of 16 bytes).
+// loads are 16-byte aligned (the bases 16-byte aligned, B rows of a multiple of 16 bytes).
 template <typename T>
 inline bool crg_supported(const void* A, long lda, long a_rows, const void* B, long ldb,
                           long b_rows) {
@@ -254,7 +220,7 @@ inline void crg_split(int M, int N, int K, int RB, int CB, int& ksplit, int& kch
 // Whether the register-tiled kernel suits a product whose M x N outputs, in ksplit K slices,
 // form the 16 RB x 16 CB wavefront tiles: below half a round of the machine's 1024 wavefront
 // slots its 64-row tiles leave most SIMDs idle and the LDS-staged engine's smaller tuned tiles
-// are faster (vHS at N = 200, M = 1600 and 128 walkers: 360 tiles).
+// are faster.
 inline bool crg_fills(int M, int N, int RB, int CB, int ksplit = 1) {
   constexpr long kMinTiles = 512;
   return (long)ceil_div(M, 16 * RB) * ceil_div(N, 16 * CB) * ksplit >= kMinTiles;

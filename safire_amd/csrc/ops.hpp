@@ -131,6 +131,12 @@ struct Rotated {
   float* Lnak_r32 = nullptr;  // FP32 real part (mixed precision, real determinant)
   c32* Lnak32 = nullptr;      // FP32 copy (mixed precision, complex determinant)
   bool real = false;
+  // mixed precision, real determinant: Lnak_r32 split into bfloat16 pieces and packed for vbias
+  // (split3.hpp, one block per spin at s3_off); null when it does not apply
+  char* Lnak_s3 = nullptr;
+  size_t s3_off[2] = {0, 0};
+  // and packed for the fused exchange (exchange.hip; electrons <= 40), one block per spin
+  char* Lexx_s3[2] = {nullptr, nullptr};
 };
 
 class CholeskyOps {
@@ -168,8 +174,8 @@ class CholeskyOps {
   // v[w][m] = sqrt(dt) c sum_{a,k} G[w][a][k] Lnak[m][a][k]   (vbias, :328-428)
   // prec == kMixed runs the contraction in FP32 and writes FP64 v.
   void vbias(const z64* G, int W, double dt, z64* v, Precision prec) const;
-  // vbias of a complex64 copy of G (FP32 MFMA; the same values as vbias(G, ..., kMixed), which
-  // rounds G to FP32 while staging it)
+  // vbias of a complex64 copy of G (the same values as vbias(G, ..., kMixed), which rounds G to FP32
+  // first)
   void vbias32(const c32* G, int W, double dt, z64* v) const;
   // V[s][w][i][k] = sqrt(dt) sum_m L_s[i][k][m] X[w][m] for the nspin_L() blocks s (vHS,
   // :282-326, [nstot][nwalk][NMO][NMO]); V is z64 (FP64) or c32
@@ -193,7 +199,8 @@ class CholeskyOps {
   void release(Rotated& r) const;
   // the hamiltonian's own determinant
   Rotated self() const {
-    return Rotated{PsiT_, Lnak_, haj_, Lnak_r_, Lnak_r32_, Lnak32_, real_trial_};
+    return Rotated{PsiT_, Lnak_, haj_, Lnak_r_, Lnak_r32_, Lnak32_, real_trial_, Lnak_s3_,
+                   {s3_off_[0], s3_off_[1]}, {Lexx_s3_[0], Lexx_s3_[1]}};
   }
   // vMF (NOMSD.cpp:437-464) with the charge-decomposition zero_imag (AFQMCBasePropagator.cpp:105)
   void vMF(double dt, z64* v) const;
@@ -222,15 +229,29 @@ class CholeskyOps {
   float* Lnak_r32_ = nullptr;
   c32* Lnak32_ = nullptr;
   z64* haj_ = nullptr;      // [nel][N]
+  // mixed precision: operands split into bfloat16 pieces and packed (split3.hpp).  Lpair_s3_ [nl]:
+  // the rows L[i][k] of the orbital pairs i <= k in the order of pairs_ (i << 16 | k); null where the
+  // tensor does not qualify (not symmetric, not finite, beyond the 32-bit offsets).
+  char* Lpair_s3_ = nullptr;
+  uint32_t* pairs_ = nullptr;
+  char* Lnak_s3_ = nullptr;
+  size_t s3_off_[2] = {0, 0};
+  char* Lexx_s3_[2] = {nullptr, nullptr};
+  void build_pairs();
+  // packs the FP32 half-rotated tensor for vbias and the exchange (split3.hpp)
+  void build_split(Rotated& r) const;
   void free_all();
   void exchange_spin(int sp, const z64* Gblk, int W, z64* part, z64* Kl, Precision prec,
                      const Rotated& t) const;
   void half_rotate_into(const z64* PsiT, Rotated& r) const;
   static bool crg_path();
+  // the force bias in FP32 from G in FP64 or already rounded to FP32
+  template <typename TG>
+  void vbias_f32(const cplx<TG>* G, int W, double dt, z64* v) const;
   // the fused on-chip exchange applies (FP32, real half-rotated tensor, n <= 40)
-  bool exchange_fused_path(Precision prec, bool real = true) const;
+  bool exchange_fused_path(Precision prec, const Rotated& t) const;
   // exchange partials per walker and spin block of the chosen path
-  int exchange_parts(Precision prec, bool real = true) const;
+  int exchange_parts(Precision prec, const Rotated& t) const;
 };
 
 // ---------------------------------------------------------------------------------------------

@@ -1,0 +1,156 @@
+"""The mixed-precision contractions on the bfloat16 matrix cores (split3.hpp) against FP64.
+
+Every FP32 operand is split exactly into three bfloat16 pieces and the six partial products above
+2^-24 are summed in FP32.  The result differs from the FP64 sum of the FP32-rounded operands by
+at most (S = sum |a b|, u = 2^-24, G = ceil(K / 32) groups):
+  * the partial products left out: |a1 b2| + |a2 b1| + |a2 b2| <= (2^-8 2^-16 2 + 2^-32) |a b| < 3 u S
+  * the FP32 additions: within a group at most 192 roundings of a partial sum of that group, one
+    of the accumulator per group: (192 + G) u S
+  * K slices summed in FP64 and rounded once, the scale factor's product: 2 u |result|
+so |error| <= (200 + G) u S, element by element.  The sizes put walkers, pairs, vectors and k values
+on and off the 16-row, 32/16 x 64..96 tile and 32-k group edges.
+"""
+import os
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+from safire_amd.synthetic import make_problem  # noqa: E402
+
+U = 2.0 ** -24
+
+
+@pytest.fixture(scope="module")
+def gpu():
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from safire_amd import afq
+    return afq, afq.Context(0), torch
+
+
+def f32(x):
+    return np.asarray(x).astype(np.complex64 if np.iscomplexobj(x) else np.float32)
+
+
+def bound(A, B, K):
+    """(200 + G) u sum |a b| of each output, A [W][K] complex, B [n][K] real."""
+    g = (200 + (K + 31) // 32) * U
+    return g * (np.abs(A.real) @ np.abs(B).T), g * (np.abs(A.imag) @ np.abs(B).T)
+
+
+# tile edges: 16 and 32 walkers, 64 / 80 / 96 columns, 32 k values; the smallest and ragged sizes
+@pytest.mark.parametrize("N,M,W", [(2, 1, 1), (8, 31, 15), (9, 32, 16), (13, 33, 17), (16, 64, 33),
+                                   (24, 96, 64), (31, 155, 65), (97, 487, 301), (200, 160, 130)])
+def test_vhs(gpu, N, M, W):
+    afq, ctx, torch = gpu
+    print(f"case: split vHS N={N} M={M} W={W}", flush=True)
+    p = make_problem(N, 1, M, 3)
+    ham = afq.HamiltonianOperations(ctx, p.h1, p.Likn, p.PsiT, 1, precision=afq.AFQ_MIXED)
+    rng = np.random.default_rng(W)
+    X = f32(rng.normal(size=(W, M)) + 1j * rng.normal(size=(W, M)))
+    V = afq.empty((W, N, N), torch.complex64)
+    ham.vHS(afq.device_tensor(X), V, 1.0)
+    V = afq.host(V)
+    assert np.array_equal(V, np.transpose(V, (0, 2, 1)))
+    B = f32(p.Likn).reshape(N * N, M).astype(np.float64)
+    A = X.astype(np.complex128)
+    ref, (br, bi) = A @ B.T, bound(A, B, M)
+    d = V.reshape(W, -1) - ref
+    assert np.all(np.abs(d.real) <= br) and np.all(np.abs(d.imag) <= bi)
+
+
+@pytest.mark.parametrize("N,n,nd,M,W", [(2, 1, 0, 1, 1), (9, 2, 0, 33, 17), (16, 3, 2, 95, 31),
+                                        (40, 7, 0, 161, 64), (33, 8, 0, 165, 129),
+                                        (120, 30, 28, 97, 160)])
+def test_vbias(gpu, N, n, nd, M, W):
+    afq, ctx, torch = gpu
+    print(f"case: split vbias N={N} n={n}+{nd} M={M} W={W}", flush=True)
+    p = make_problem(N, n, M, 4)
+    wt = afq.AFQ_COLLINEAR if nd else afq.AFQ_CLOSED
+    rows = np.concatenate([p.PsiT, p.PsiT[:nd]])
+    ham = afq.HamiltonianOperations(ctx, p.h1, p.Likn, rows, n, nd, walker_type=wt,
+                                    precision=afq.AFQ_MIXED)
+    rng = np.random.default_rng(N)
+    G = rng.normal(size=(W, n + nd, N)) + 1j * rng.normal(size=(W, n + nd, N))
+    v = afq.empty((W, M), torch.complex128)
+    ham.vbias(afq.device_tensor(G), v, 1.0)
+    v = afq.host(v)
+    L = ham.tensors()[0].real
+    c = 1.0 if nd else 2.0
+    ref, br, bi, g0, l0 = 0, 0, 0, 0, 0
+    for ns in (n, nd):
+        if not ns:
+            continue
+        A = f32(G[:, g0:g0 + ns].reshape(W, -1)).astype(np.complex128)
+        B = f32(L[l0:l0 + M * ns * N].reshape(M, -1)).astype(np.float64)
+        r, i = bound(A, B, ns * N)
+        ref, br, bi = ref + c * (A @ B.T), br + c * r, bi + c * i
+        g0, l0 = g0 + ns, l0 + M * ns * N
+    d = v - ref
+    assert np.all(np.abs(d.real) <= br) and np.all(np.abs(d.imag) <= bi)
+
+
+def test_infinities_and_nan(gpu):
+    """A walker with an infinite or NaN field gives the infinities and NaN of the FP32 products
+    (AFQ_CRGEMM=0); the other walkers keep their bits."""
+    afq, ctx, torch = gpu
+    N, M, W = 12, 40, 21
+    print(f"case: split vHS with infinities N={N} M={M} W={W}", flush=True)
+    p = make_problem(N, 1, M, 5)
+    ham = afq.HamiltonianOperations(ctx, p.h1, p.Likn, p.PsiT, 1, precision=afq.AFQ_MIXED)
+    rng = np.random.default_rng(1)
+    X = f32(rng.normal(size=(W, M)) + 1j * rng.normal(size=(W, M)))
+
+    def vhs(x):
+        V = afq.empty((W, N, N), torch.complex64)
+        ham.vHS(afq.device_tensor(x), V, 1.0)
+        return afq.host(V)
+    clean = vhs(X)
+    Y = X.copy()
+    Y[3, 7] = np.inf
+    Y[16, 39] = complex(0.5, -np.inf)
+    Y[18, 0] = np.nan
+    Y[20, 5], Y[20, 6] = np.inf, -np.inf
+    got = vhs(Y)
+    os.environ["AFQ_CRGEMM"] = "0"
+    try:
+        ref = vhs(Y)
+    finally:
+        del os.environ["AFQ_CRGEMM"]
+    rest = [w for w in range(W) if w not in (3, 16, 18, 20)]
+    assert np.array_equal(got[rest], clean[rest])
+    for part in (np.real, np.imag):
+        g, r = part(got), part(ref)
+        assert np.array_equal(np.isnan(g), np.isnan(r))
+        inf = np.isinf(r)
+        assert np.array_equal(np.isinf(g), inf) and np.array_equal(g[inf], r[inf])
+
+
+def test_tensors_outside_the_split_keep_the_fp32_product(gpu):
+    """A Cholesky tensor with an infinity is contracted as before (no split operand is built)."""
+    afq, ctx, torch = gpu
+    N, M, W = 10, 33, 5
+    print("case: infinite Cholesky entry", flush=True)
+    p = make_problem(N, 1, M, 6)
+    L = p.Likn.copy()
+    L[2, 4, 9] = L[4, 2, 9] = np.inf
+    ham = afq.HamiltonianOperations(ctx, p.h1, L, p.PsiT, 1, precision=afq.AFQ_MIXED)
+    X = f32(np.ones((W, M)) * (1 + 2j))
+
+    def vhs():
+        V = afq.empty((W, N, N), torch.complex64)
+        ham.vHS(afq.device_tensor(X), V, 1.0)
+        return afq.host(V)
+    V = vhs()
+    os.environ["AFQ_CRGEMM"] = "0"
+    try:
+        ref = vhs()
+    finally:
+        del os.environ["AFQ_CRGEMM"]
+    assert np.array_equal(V, ref, equal_nan=True)
+    assert not np.any(np.isfinite(V[:, 2, 4])) and not np.any(np.isfinite(V[:, 4, 2]))
+    V[:, 2, 4] = V[:, 4, 2] = 0
+    assert np.all(np.isfinite(V))
