@@ -994,6 +994,7 @@ void propagate(Context& c, const PropagateArgs& a) {
     propagate_t<double>(c, a);
   } else {
     AFQ_CHECK(a.P1r32 || a.P1c32, kErrArg, "FP32 P1 missing");
+    if (a.fused && propagate_split(c, a)) return;
     propagate_t<float>(c, a);
   }
 }

@@ -112,6 +112,9 @@ struct PropagateArgs {
   bool v_symmetric = false;  // V[i][j] == V[j][i] exactly (vHS output): lets 'H' use the fused kernel
 };
 void propagate(Context& c, const PropagateArgs& a);
+// The mixed-precision propagation in one launch on the bfloat16 matrix cores (prop_split.hip), for
+// TA = 'N' and N <= 256; false when the shape or the arguments are outside it.
+bool propagate_split(Context& c, const PropagateArgs& a);
 // orthogonalize (orthogonalize.hpp:131-169): Phi <- Q with Phi = Q R, R upper triangular with a
 // positive real diagonal (Cholesky-QR2); ldet += log det R.
 void orthogonalize(Context& c, z64* Phi, long phi_bs, int W, int N, int n, z64* ldet);
