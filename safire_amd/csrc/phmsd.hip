@@ -375,48 +375,46 @@ struct EpiStoreWL {
   }
 };
 
-// jr[w][n] = sum_i T[i][i] (Jref), tz[w][n] = sum_ik T[k][i] T[i][k] over the reference rows.
-__global__ void k_ph_energy_prep(int W, int NS, int nel, int nact, const z64* __restrict__ T3,
-                                 z64* __restrict__ jr, z64* __restrict__ tz) {
-  const long slice = (long)nact * nel;
-  const long wn = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (wn >= (long)W * NS) return;
-  const z64* T = T3 + wn * slice;
-  z64 j = {0.0, 0.0}, z = {0.0, 0.0};
-  for (int i = 0; i < nel; ++i) {
-    j = zadd(j, T[i * nel + i]);
-    for (int k = 0; k < nel; ++k) z = zfma(T[k * nel + i], T[i * nel + k], z);
+// dst[to(t)] = *from(t) for t < count by 256 threads, eight loads in flight a thread
+template <typename From, typename To>
+__device__ inline void stage_lds(z64* dst, int count, From from, To to) {
+  for (int t0 = threadIdx.x; t0 < count; t0 += 8 * 256) {
+    z64 v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = *from(min(t0 + 256 * i, count - 1));
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (t0 + 256 * i < count) dst[to(t0 + 256 * i)] = v[i];
   }
-  jr[wn] = j;
-  tz[wn] = z;
 }
-
-// Excitations of rank R, configurations [u0, u1), slices [n0, n0 + nc) of walker w. With
-// g_p[l] = sum_q Minv[p][q] V[x_q][l] the excited Y differs from the reference Zref = T[0:nel]
-// only in the hole rows, Y[h_p] = Zref[h_p] + g_p, hence
-//   Kn = Jref + sum_p g_p[h_p],   eX = sum_pq g_p[h_q] g_q[h_p] + 2 sum_pl g_p[l] T[l][h_p],
-// which are tr(Y) and tr(Y^2) - tr(Zref^2) of the reference's per-determinant evaluation.
-// When there are fewer excitations than threads, G threads share an excitation and take every
-// G-th slice; their sums are combined in a fixed order.
-// part [W][nch][nconf][3] <- (e1 on the haj slice, sum eX, sum Kn^2 - Jref^2); KE [W][nconf][M].
+// One slice T (an nact x nel matrix; Zref its rows [0, nel)) and one excitation of rank R.  With
+// V[x] = T[x] - QQ0[x] Zref for the particle rows and g_p[l] = sum_q Minv[p][q] V[x_q][l] the
+// excited Y differs from Zref only in the hole rows, Y[h_p] = Zref[h_p] + g_p, hence
+//   Kn = Jref + sum_p g_p[h_p],   eX = sum_pq g_p[h_q] g_q[h_p] + 2 sum_pl g_p[l] Zref[l][h_p],
+// which are tr(Y) and tr(Y^2) - tr(Zref^2) of the reference's per-determinant evaluation.  The last
+// sum is 2 sum_pq Minv[p][q] U[x_q][h_p] with U = V Zref, which no excitation changes: a slice
+// forms it once and an excitation multiplies R x R blocks only.
 template <int R>
-__device__ inline void ph_slice_terms(const z64* __restrict__ Ts, int nel, const int (&h)[R],
-                                      const int (&x)[R], const z64 (&Mi)[R][R], z64& k, z64& ex) {
+__device__ inline void ph_slice_terms(const z64* __restrict__ V, const z64* __restrict__ U,
+                                      const int (&h)[R], const int (&xo)[R],
+                                      const z64 (&Mi)[R][R], z64& k, z64& ex) {
   z64 gh[R][R];
   z64 acc = {0.0, 0.0};
-  for (int l = 0; l < nel; ++l) {
-    z64 V[R];
 #pragma unroll
-    for (int q = 0; q < R; ++q) V[q] = Ts[x[q] * nel + l];
+  for (int p = 0; p < R; ++p)
+#pragma unroll
+    for (int q = 0; q < R; ++q) acc = zfma(Mi[p][q], U[xo[q] + h[p]], acc);
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    z64 v[R];  // V[x_r][h_q]
+#pragma unroll
+    for (int r = 0; r < R; ++r) v[r] = V[xo[r] + h[q]];
 #pragma unroll
     for (int p = 0; p < R; ++p) {
       z64 g = {0.0, 0.0};
 #pragma unroll
-      for (int q = 0; q < R; ++q) g = zfma(Mi[p][q], V[q], g);
-      acc = zfma(g, Ts[l * nel + h[p]], acc);
-#pragma unroll
-      for (int q = 0; q < R; ++q)
-        if (h[q] == l) gh[p][q] = g;
+      for (int r = 0; r < R; ++r) g = zfma(Mi[p][r], v[r], g);
+      gh[p][q] = g;
     }
   }
   k = {0.0, 0.0};
@@ -429,63 +427,52 @@ __device__ inline void ph_slice_terms(const z64* __restrict__ Ts, int nel, const
   }
 }
 
+// The slices [n0, n0 + nc) of walker w in LDS and where their excitations go
+struct PhSlices {
+  int nel, nconf, M, n0, nc, SL, vofs, uofs;
+  const z64* T;  // LDS [nc][SL]: slice, V at vofs, U at uofs
+  const z64* j;  // LDS [nc]: Jref
+  z64* red;      // LDS [256][3]
+  const int *exc, *mstart;
+  const z64* Minv;  // this walker's
+  z64 *part, *KE;   // this walker's (and run of slices')
+};
+
+// Excitations of rank R, configurations [u0, u1).  When there are fewer excitations than threads, G
+// threads share an excitation and take every G-th slice; their sums are combined in a fixed order.
 template <int R>
-__global__ void __launch_bounds__(256)
-    k_ph_energy_rank(int nel, int nact, int nconf, int M, int NS, int NC, int u0, int u1,
-                     const int* __restrict__ exc, const int* __restrict__ mstart, int P2,
-                     const z64* __restrict__ T3, const z64* __restrict__ Qv,
-                     const z64* __restrict__ jr, const z64* __restrict__ Minv,
-                     z64* __restrict__ part, z64* __restrict__ KE) {
-  extern __shared__ z64 smem[];
-  const int slice = nact * nel, nvir = nact - nel;
-  const int chunk = blockIdx.x, w = blockIdx.y, nch = gridDim.x;
-  const int n0 = chunk * NC, nc = min(NC, NS - n0);
-  z64* red = smem + (long)NC * slice;   // [256][3]
-  z64* sq = red + 3 * 256;              // [nvir][nel] QQ0 rows of the particles
-  const z64* src = T3 + ((long)w * NS + n0) * slice;
-  for (int t = threadIdx.x; t < nc * slice; t += 256) smem[t] = src[t];
-  for (int t = threadIdx.x; t < nvir * nel; t += 256) sq[t] = Qv[(long)w * nvir * nel + t];
-  __syncthreads();
-  // particle rows x >= nel become V[x][l] = T[x][l] - sum_i QQ0[x][i] T[i][l] (the reference
-  // rows are only read)
-  for (int t = threadIdx.x; t < nc * nvir * nel; t += 256) {
-    const int l = t % nel, x = (t / nel) % nvir, c = t / (nvir * nel);
-    z64* T = smem + (long)c * slice;
-    z64 b = {0.0, 0.0};
-    for (int i = 0; i < nel; ++i) b = zfma(sq[x * nel + i], T[i * nel + l], b);
-    T[(nel + x) * nel + l] = zsub(T[(nel + x) * nel + l], b);
-  }
-  __syncthreads();
-  const z64* jw = jr + (long)w * NS + n0;
+__device__ inline void ph_rank(const PhSlices& a, int u0, int u1) {
   const int cnt = u1 - u0;
-  const int G = cnt >= 256 ? 1 : max(1, min(nc, 256 / cnt));
+  if (cnt <= 0) return;
+  const int G = cnt >= 256 ? 1 : max(1, min(a.nc, 256 / cnt));
   const int nitem = cnt >= 256 ? cnt : cnt * G;
   for (int it0 = 0; it0 < nitem; it0 += 256) {
     const int it = it0 + threadIdx.x;
     z64 a0 = {0.0, 0.0}, a1 = {0.0, 0.0}, a2 = {0.0, 0.0};
     if (it < nitem) {
       const int u = u0 + it / G, g = it % G;
-      const int* e = exc + (long)u * kXS;
-      const z64* mi = Minv + (long)w * P2 + mstart[u];
-      int h[R], x[R];
+      const int* e = a.exc + (long)u * kXS;
+      const z64* mi = a.Minv + a.mstart[u];
+      int h[R], xo[R];
       z64 Mi[R][R];
 #pragma unroll
       for (int p = 0; p < R; ++p) {
         h[p] = e[p];
-        x[p] = e[R + p];
+        xo[p] = (e[R + p] - a.nel) * a.nel;
 #pragma unroll
         for (int q = 0; q < R; ++q) Mi[p][q] = mi[p * R + q];
       }
-      z64* ke = KE + ((long)w * nconf + u) * M;
-      for (int c = g; c < nc; c += G) {
+      z64* ke = a.KE + (long)u * a.M;
+      for (int c = g; c < a.nc; c += G) {
         z64 k, ex;
-        ph_slice_terms<R>(smem + (long)c * slice, nel, h, x, Mi, k, ex);
-        const int n = n0 + c;
-        if (n < M) {
-          const z64 kn = zadd(jw[c], k);
+        const z64* T = a.T + (long)c * a.SL;
+        ph_slice_terms<R>(T + a.vofs, T + a.uofs, h, xo, Mi, k, ex);
+        const int n = a.n0 + c;
+        if (n < a.M) {
+          const z64 kn = zadd(a.j[c], k);
           ke[n] = kn;
           a1 = zadd(a1, ex);
-          a2 = zadd(a2, zsub(zmul(kn, kn), zmul(jw[c], jw[c])));
+          a2 = zadd(a2, zsub(zmul(kn, kn), zmul(a.j[c], a.j[c])));
         } else {
           a0 = zadd(a0, k);
         }
@@ -493,25 +480,26 @@ __global__ void __launch_bounds__(256)
     }
     if (G == 1) {
       if (it < nitem) {
-        z64* pw = part + (((long)w * nch + chunk) * nconf + u0 + it) * 3;
+        z64* pw = a.part + (long)(u0 + it) * 3;
         pw[0] = a0;
         pw[1] = a1;
         pw[2] = a2;
       }
     } else {
-      red[3 * threadIdx.x + 0] = a0;
-      red[3 * threadIdx.x + 1] = a1;
-      red[3 * threadIdx.x + 2] = a2;
+      __syncthreads();  // (the last rank's sums are read)
+      a.red[3 * threadIdx.x + 0] = a0;
+      a.red[3 * threadIdx.x + 1] = a1;
+      a.red[3 * threadIdx.x + 2] = a2;
       __syncthreads();
       if ((int)threadIdx.x < cnt) {
         z64 s0 = {0.0, 0.0}, s1 = {0.0, 0.0}, s2 = {0.0, 0.0};
         for (int g = 0; g < G; ++g) {
-          const z64* r = red + 3 * (threadIdx.x * G + g);
+          const z64* r = a.red + 3 * (threadIdx.x * G + g);
           s0 = zadd(s0, r[0]);
           s1 = zadd(s1, r[1]);
           s2 = zadd(s2, r[2]);
         }
-        z64* pw = part + (((long)w * nch + chunk) * nconf + u0 + threadIdx.x) * 3;
+        z64* pw = a.part + (long)(u0 + threadIdx.x) * 3;
         pw[0] = s0;
         pw[1] = s1;
         pw[2] = s2;
@@ -520,13 +508,91 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-// KE[w][0][n] = Jref for n < M (the reference configuration's Coulomb vector)
-__global__ void k_ph_ke_ref(int W, int M, int NS, int nconf, const z64* __restrict__ jr,
-                            z64* __restrict__ KE) {
-  long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (long)W * M) return;
-  const int w = (int)(t / M), n = (int)(t % M);
-  KE[(long)w * nconf * M + n] = jr[(long)w * NS + n];
+struct PhRanks {
+  int off[8];  // configurations of rank r: [off[r], off[r + 1])
+};
+
+// Every configuration's terms over the slices [n0, n0 + nc) of walker w (the slices staged in LDS
+// once for all ranks).
+//   jr[w][n] = sum_i T[i][i] (Jref), tz[w][n] = sum_ik T[k][i] T[i][k] over the reference rows;
+//   part [W][nch][nconf][3] <- (e1 on the haj slice, sum eX, sum Kn^2 - Jref^2);
+//   KE [W][nconf][M] <- the Coulomb vectors (configuration 0: Jref).
+// Bound by FP64 vector products (45 complex ones for an excitation of rank 3 and a slice) and by the
+// reading of T.  256 walkers, 321 slices, 15 x 10 active orbitals, 2000 determinants, both spins: a
+// kernel per rank with the sum over l in it and one for jr and tz 2.6 ms, this kernel 0.80 ms.
+// RMAX: the largest rank (4 keeps two workgroups a CU within the register file).
+template <int RMAX>
+__global__ void __launch_bounds__(256, RMAX <= 4 ? 2 : 1)
+    k_ph_energy_exc(int nel, int nact, int nconf, int M, int NS, int NC, PhRanks ranks,
+                    const int* __restrict__ exc, const int* __restrict__ mstart, int P2,
+                    const z64* __restrict__ T3, const z64* __restrict__ Qv,
+                    const z64* __restrict__ Minv, z64* __restrict__ jr, z64* __restrict__ tz,
+                    z64* __restrict__ part, z64* __restrict__ KE) {
+  extern __shared__ z64 smem[];
+  __shared__ z64 sj[32];
+  const int slice = nact * nel, nvir = nact - nel, SL = slice + nvir * nel, tid = threadIdx.x;
+  const int chunk = blockIdx.x, w = blockIdx.y, nch = gridDim.x;
+  const int n0 = chunk * NC, nc = min(NC, NS - n0);
+  z64* red = smem + (long)NC * SL;  // [256][3]
+  z64* sq = red + 3 * 256;          // [nvir][nel] QQ0 rows of the particles
+  const z64* src = T3 + ((long)w * NS + n0) * slice;
+  stage_lds(smem, nc * slice, [&](int t) { return src + t; },
+            [&](int t) { return t / slice * SL + t % slice; });
+  for (int t = tid; t < nvir * nel; t += 256) sq[t] = Qv[(long)w * nvir * nel + t];
+  __syncthreads();
+  {  // eight lanes a slice (NC <= 32)
+    const int c = tid >> 3;
+    z64 j = {0.0, 0.0}, z = {0.0, 0.0};
+    if (c < nc) {
+      const z64* T = smem + (long)c * SL;
+      for (int i = tid & 7; i < nel; i += 8) {
+        j = zadd(j, T[i * nel + i]);
+        for (int k = 0; k < nel; ++k) z = zfma(T[k * nel + i], T[i * nel + k], z);
+      }
+    }
+#pragma unroll
+    for (int off = 4; off > 0; off >>= 1) {
+      j = zadd(j, z64{__shfl_xor(j.re, off, 64), __shfl_xor(j.im, off, 64)});
+      z = zadd(z, z64{__shfl_xor(z.re, off, 64), __shfl_xor(z.im, off, 64)});
+    }
+    if (c < nc && (tid & 7) == 0) {
+      const int n = n0 + c;
+      sj[c] = j;
+      jr[(long)w * NS + n] = j;
+      tz[(long)w * NS + n] = z;
+      if (n < M) KE[(long)w * nconf * M + n] = j;
+    }
+  }
+  // particle rows x >= nel become V[x][l] = T[x][l] - sum_i QQ0[x][i] T[i][l] (the reference
+  // rows are only read)
+  for (int t = tid; t < nc * nvir * nel; t += 256) {
+    const int l = t % nel, x = (t / nel) % nvir, c = t / (nvir * nel);
+    z64* T = smem + (long)c * SL;
+    z64 b = {0.0, 0.0};
+    for (int i = 0; i < nel; ++i) b = zfma(sq[x * nel + i], T[i * nel + l], b);
+    T[(nel + x) * nel + l] = zsub(T[(nel + x) * nel + l], b);
+  }
+  __syncthreads();
+  // U[x][h] = sum_l V[x][l] T[l][h]
+  for (int t = tid; t < nc * nvir * nel; t += 256) {
+    const int h = t % nel, x = (t / nel) % nvir, c = t / (nvir * nel);
+    z64* T = smem + (long)c * SL;
+    z64 b = {0.0, 0.0};
+    for (int l = 0; l < nel; ++l) b = zfma(T[(nel + x) * nel + l], T[l * nel + h], b);
+    T[slice + x * nel + h] = b;
+  }
+  __syncthreads();
+  const PhSlices a{nel, nconf, M, n0, nc, SL, nel * nel, slice, smem, sj, red, exc, mstart,
+                   Minv + (long)w * P2, part + ((long)w * nch + chunk) * nconf * 3,
+                   KE + (long)w * nconf * M};
+  ph_rank<1>(a, ranks.off[1], ranks.off[2]);
+  ph_rank<2>(a, ranks.off[2], ranks.off[3]);
+  ph_rank<3>(a, ranks.off[3], ranks.off[4]);
+  ph_rank<4>(a, ranks.off[4], ranks.off[5]);
+  if constexpr (RMAX > 4) {
+    ph_rank<5>(a, ranks.off[5], ranks.off[6]);
+    ph_rank<6>(a, ranks.off[6], ranks.off[7]);
+  }
 }
 
 // Opposite-spin Coulomb coupling over Cholesky slices [n0, n0 + CH) of walker w:
@@ -544,34 +610,48 @@ __global__ void __launch_bounds__(256)
   const int n0 = chunk * CH, cn = min(CH, M - n0);
   const z64* Ka = KEa + (long)w * na * M;
   const z64* Kb = KEb + (long)w * nb * M;
-  // slices in LDS ([na][CH] then [nb][CH]) when they fit, else read in place
+  // slices in LDS ([na][CH + 1] then [nb][CH + 1]) when they fit, else read in place
   const z64* sa = Ka + n0;
   const z64* sb = Kb + n0;
   long ld = M;
   if (lds) {
     z64* da = sk;
-    z64* db = sk + (long)na * CH;
-    for (int t = tid; t < na * CH; t += 256) {
-      const int u = t / CH, j = t % CH;
-      da[t] = j < cn ? Ka[(long)u * M + n0 + j] : z64{0.0, 0.0};
-    }
-    for (int t = tid; t < nb * CH; t += 256) {
-      const int v = t / CH, j = t % CH;
-      db[t] = j < cn ? Kb[(long)v * M + n0 + j] : z64{0.0, 0.0};
-    }
+    z64* db = sk + (long)na * (CH + 1);
+    auto to = [&](int t) { return t + t / CH; };
+    stage_lds(da, na * CH,
+              [&](int t) { return Ka + (long)(t / CH) * M + n0 + min(t % CH, cn - 1); }, to);
+    stage_lds(db, nb * CH,
+              [&](int t) { return Kb + (long)(t / CH) * M + n0 + min(t % CH, cn - 1); }, to);
     __syncthreads();
     sa = da;
     sb = db;
-    ld = CH;
+    ld = CH + 1;
   }
   const z64* oa = ova + (long)w * na;
   const z64* ob = ovb + (long)w * nb;
   z64 acc = {0.0, 0.0};
-  for (int d = tid; d < ndet; d += 256) {
-    const int u = crow[d], v = ccol[d];
-    z64 dot = {0.0, 0.0};
-    for (int j = 0; j < cn; ++j) dot = zfma(sa[u * ld + j], sb[v * ld + j], dot);
-    acc = zfma(zmul(cval[d], zmul(oa[u], ob[v])), dot, acc);
+  // eight determinants at a time: the chain of index, weight and dot product of a single one is
+  // bound by the latency of its loads
+  constexpr int B = 8;
+  for (int d0 = tid; d0 < ndet; d0 += 256 * B) {
+    int u[B], v[B];
+    z64 wt[B], dot[B];
+#pragma unroll
+    for (int i = 0; i < B; ++i) {
+      const int d = min(d0 + 256 * i, ndet - 1);
+      u[i] = crow[d];
+      v[i] = ccol[d];
+      wt[i] = cval[d];
+      dot[i] = z64{0.0, 0.0};
+    }
+#pragma unroll
+    for (int i = 0; i < B; ++i) wt[i] = zmul(wt[i], zmul(oa[u[i]], ob[v[i]]));
+    for (int j = 0; j < cn; ++j)
+#pragma unroll
+      for (int i = 0; i < B; ++i) dot[i] = zfma(sa[u[i] * ld + j], sb[v[i] * ld + j], dot[i]);
+#pragma unroll
+    for (int i = 0; i < B; ++i)
+      if (d0 + 256 * i < ndet) acc = zfma(wt[i], dot[i], acc);
   }
   acc = block_sum<256>(acc, red);
   if (tid == 0) out[(long)w * nch + chunk] = acc;
@@ -1051,11 +1131,15 @@ void PhmsdTrial::energy(const z64* Pa, const z64* Pb, int W, z64* E, z64* Ov, lo
   z64* tz[2];
   for (int sp = 0; sp < 2; ++sp) {
     const SpinDev& d = sp_[sp];
-    const long slice = (long)d.nact * d.nel;
-    // LDS: NC slices, the [256][3] reduction buffer and the particle rows of QQ0 within 64 KB
-    const long budget = 64L * 1024 - (long)sizeof(z64) * (3 * 256 + (long)d.nvir * d.nel);
-    const int NC = (int)std::min<long>(32, budget / (slice * (long)sizeof(z64)));
-    AFQ_CHECK(NC >= 1, kErrShape, "active space too large for the PHMSD energy kernel");
+    const long slice = (long)d.nact * d.nel, vn = (long)d.nvir * d.nel, SL = slice + vn;
+    AFQ_CHECK((64L * 1024 - (long)sizeof(z64) * (3 * 256 + vn)) / (slice * (long)sizeof(z64)) >= 1,
+              kErrShape, "active space too large for the PHMSD energy kernel");
+    // LDS: NC slices with their U, the [256][3] reduction buffer and the particle rows of QQ0: two
+    // workgroups a CU, or one where a slice is too large for that
+    const long fixed = (long)sizeof(z64) * (3 * 256 + vn) + 1024;
+    long fit = (80L * 1024 - fixed) / (SL * (long)sizeof(z64));
+    if (fit < 1) fit = (160L * 1024 - fixed) / (SL * (long)sizeof(z64));
+    const int NC = (int)std::min(32L, std::max(1L, fit));
     nch[sp] = ceil_div(NS, NC);
     z64* T3 = scratch_as<z64>(ctx_, "ph_T3", (size_t)W * NS * slice);
     {  // T3[w][n][a][l] = sum_k Lext[n][a][k] GA[w][l][k]: rows (n, a), columns (w, l)
@@ -1068,45 +1152,40 @@ void PhmsdTrial::energy(const z64* Pa, const z64* Pb, int W, z64* E, z64* Ov, lo
     jr[sp] = scratch_as<z64>(ctx_, tag("ph_jr", sp), (size_t)W * NS);
     tz[sp] = scratch_as<z64>(ctx_, tag("ph_tz", sp), (size_t)W * NS);
     const z64* Qv = scratch_as<z64>(ctx_, tag("ph_Qv", sp), (size_t)W * std::max(d.nvir, 1) * d.nel);
-    hipLaunchKernelGGL(k_ph_energy_prep, dim3(ceil_div((long)W * NS, 256)), dim3(256), 0, s, W, NS,
-                       d.nel, d.nact, T3, jr[sp], tz[sp]);
-    AFQ_LAUNCH_CHECK();
     part[sp] = scratch_as<z64>(ctx_, tag("ph_part", sp), (size_t)W * nch[sp] * d.nconf * 3);
     KE[sp] = scratch_as<z64>(ctx_, tag("ph_KE", sp), (size_t)W * M * d.nconf);
-    hipLaunchKernelGGL(k_ph_ke_ref, dim3(ceil_div((long)W * M, 256)), dim3(256), 0, s, W, M, NS,
-                       d.nconf, jr[sp], KE[sp]);
-    AFQ_LAUNCH_CHECK();
     const z64* Mi = scratch_as<z64>(ctx_, tag("ph_Minv", sp), (size_t)W * std::max(d.P2, 1));
-    const size_t shm = sizeof(z64) * ((size_t)NC * slice + 3 * 256 + (size_t)d.nvir * d.nel);
-    for (int r = 1; r <= d.rmax; ++r) {
-      const int u0 = d.rank_off[r], u1 = d.rank_off[r + 1];
-      if (u1 <= u0) continue;
-      dim3 g(nch[sp], W);
-#define AFQ_ERANK(R)                                                                           \
-  hipLaunchKernelGGL(k_ph_energy_rank<R>, g, dim3(256), shm, s, d.nel, d.nact, d.nconf, M, NS, \
-                     NC, u0, u1, d.exc, d.mstart, d.P2, T3, Qv, jr[sp], Mi, part[sp], KE[sp])
-      switch (r) {
-        case 1: AFQ_ERANK(1); break;
-        case 2: AFQ_ERANK(2); break;
-        case 3: AFQ_ERANK(3); break;
-        case 4: AFQ_ERANK(4); break;
-        case 5: AFQ_ERANK(5); break;
-        default: AFQ_ERANK(6); break;
-      }
-#undef AFQ_ERANK
-      AFQ_LAUNCH_CHECK();
-    }
+    const size_t shm = sizeof(z64) * ((size_t)NC * SL + 3 * 256 + (size_t)vn);
+    PhRanks ranks;
+    for (int r = 0; r < 8; ++r) ranks.off[r] = d.rank_off[std::min(r, d.rmax + 1)];
+    auto go = [&](auto kern) {
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
+      hipLaunchKernelGGL(kern, dim3(nch[sp], W), dim3(256), shm, s, d.nel, d.nact, d.nconf, M, NS,
+                         NC, ranks, d.exc, d.mstart, d.P2, T3, Qv, Mi, jr[sp], tz[sp], part[sp],
+                         KE[sp]);
+    };
+    if (d.rmax <= 4) go(k_ph_energy_exc<4>);
+    else go(k_ph_energy_exc<6>);
+    AFQ_LAUNCH_CHECK();
   }
   // opposite-spin Coulomb term over Cholesky chunks of CH slices
   const int na = sp_[0].nconf, nb = sp_[1].nconf;
-  // (both spins' slices of a chunk in 64 KB of LDS; read in place for larger expansions)
-  const int CHl = (int)std::min<long>(16, (64L * 1024) / ((long)sizeof(z64) * (na + nb)));
-  const int use_lds = CHl >= 1 ? 1 : 0;
-  const int CH = use_lds ? CHl : 16;
+  // (both spins' slices of a chunk in LDS, two workgroups a CU; read in place for larger
+  // expansions).  CH a power of two: rows of KE are read in whole 128-byte lines.  The LDS rows are
+  // one longer, or every determinant's j-th value would lie on two of the sixteen 16-byte bank
+  // groups.  Bound by the staging of KE; with the determinants eight at a time 256 walkers of 2000
+  // determinants take 416 us, one at a time and unpadded rows of 8 441 us.
+  const long fit = (76L * 1024) / ((long)sizeof(z64) * (na + nb));
+  const int use_lds = fit >= 2 ? 1 : 0;
+  int CH = 16;
+  while (use_lds && CH + 1 > fit) CH /= 2;
   const int ncross = ceil_div(M, CH);
   z64* cross = scratch_as<z64>(ctx_, "ph_cross", (size_t)W * ncross);
+  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k_ph_cross),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, 76 * 1024);
   hipLaunchKernelGGL(k_ph_cross, dim3(ncross, W), dim3(256),
-                     use_lds ? sizeof(z64) * (size_t)(na + nb) * CH : 0, s, na, nb, M, CH,
+                     use_lds ? sizeof(z64) * (size_t)(na + nb) * (CH + 1) : 0, s, na, nb, M, CH,
                      use_lds, ndet_, crow_, sp_[0].ccol, sp_[0].cval,
                      scratch_as<z64>(ctx_, "ph_ovr0", (size_t)W * na),
                      scratch_as<z64>(ctx_, "ph_ovr1", (size_t)W * nb), KE[0], KE[1], cross);
