@@ -31,14 +31,11 @@ DT, ORDER, ORTHO = 0.005, 6, 5
 SEED = 1003
 AMPLITUDE = 0.1          # Cholesky amplitude of the headline workload
 RECIPE_AMPLITUDE = 0.5   # the generator's default
-PEAK = {"fp32": 157.3e12, "fp64": 78.6e12}
+# "mixed": an FP32 product is six bfloat16 products on the matrix cores (dense peak 2.5 PFLOP/s)
+PEAK = {"mixed": 2.5e15 / 6, "fp64": 78.6e12}
 HBM_PEAK = 8.0e12
-# HBM bytes of one FP32 vHS launch (k_crgemm over the symmetric pairs) at this workload:
-# FETCH_SIZE x 2 + WRITE_SIZE x 1 in KiB (the factors that make a 1 GiB copy read and write
-# 1 GiB), rocprofv3 --pmc of `bench.py --only step`
-# (profiles/step_N200_n40_M1600_W1024_pmc.md).  Algorithmic: X 13.1 MB + L 128.6 MB + V 327.7 MB.
-VHS_TRAFFIC_BYTES = (226327 * 2 + 562803) * 1024
-VHS_ALGORITHMIC_BYTES = W * M * 8 + (N * (N + 1) // 2) * M * 4 + W * N * N * 8
+# bytes of one mixed vHS launch: X and the symmetric pairs of L as three bfloat16 pieces, V as c64
+VHS_ALGORITHMIC_BYTES = W * M * 12 + (N * (N + 1) // 2) * M * 6 + W * N * N * 8
 
 
 def flops_per_walker_step(N, n, M, K=ORDER, k_ortho=ORTHO, performed=True):
@@ -743,29 +740,28 @@ def main():
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": "c64 FP32-MFMA contractions + c128 G/LU/QR/weights",
+        "dtype": "c64 contractions (FP32 as three bfloat16 pieces) + c128 G/LU/QR/weights",
         "data": "synthetic (seeded hamiltonian, trial, fields)",
         "config": {"workload": "N=200 orbitals, 40+40 electrons, M=1600 Cholesky vectors, "
                                "1024 walkers, dt=0.005, taylor 6, QR every 5 steps",
                    "cholesky_amplitude": AMPLITUDE,
                    "precision": "mixed", "graph": "one HIP graph per step"},
         "roofline": {"bound": "mfma",
-                     "kernel": "vHS: k_crgemm, register-tiled FP32 MFMA, X [W x M] . the "
-                               "N(N+1)/2 symmetric pairs of L [M], V mirrored",
-                     "achieved": achieved / 1e12, "peak": PEAK["fp32"] / 1e12,
+                     "kernel": "vHS: k_split3_gemm, FP32 products as six bfloat16 MFMAs, X [W x M] . "
+                               "the N(N+1)/2 symmetric pairs of L [M], V mirrored",
+                     "achieved": achieved / 1e12, "peak": PEAK["mixed"] / 1e12,
                      "vhs_ms_in_eager_steps": tv * 1e3,
                      "vhs_ms_back_to_back": out["mixed"]["vhs_b2b"] * 1e3,
                      "vhs_ms_in_step_graph_events": out["mixed"]["vhs"] * 1e3,
                      "achieved_in_step_graph_events": vhs_flops / out["mixed"]["vhs"] / 1e12,
-                     "unit": "TFLOP/s", "frac": achieved / PEAK["fp32"],
-                     "traffic": VHS_TRAFFIC_BYTES,
-                     "traffic_over_algorithmic": VHS_TRAFFIC_BYTES / VHS_ALGORITHMIC_BYTES},
+                     "unit": "TFLOP/s", "frac": achieved / PEAK["mixed"],
+                     "algorithmic_bytes": VHS_ALGORITHMIC_BYTES},
         # the whole step: the FLOP the kernels issue (flops_per_walker_step) per second over the
         # MFMA peak of the contraction precision; *_all_complex: the count with every MAC
         # complex and vHS over all N^2 entries
         "step_flop_per_walker": fstep,
-        "step_roofline_frac": (fstep * W / sec) / PEAK["fp32"],
-        "step_roofline_frac_all_complex_count": (fstep_all * W / sec) / PEAK["fp32"],
+        "step_roofline_frac": (fstep * W / sec) / PEAK["mixed"],
+        "step_roofline_frac_all_complex_count": (fstep_all * W / sec) / PEAK["mixed"],
         "fp64": None if "fp64" not in out else {
             "value": W / out["fp64"]["sec"], "ms_per_step": out["fp64"]["sec"] * 1e3,
             "vhs_ms": out["fp64"]["vhs_eager"] * 1e3,
