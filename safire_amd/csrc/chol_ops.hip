@@ -98,7 +98,7 @@ CholeskyOps::CholeskyOps(Context& c, int walker_type, int N, int nup, int ndown,
       cast_f64_f32(s, (long)(nl_ * NNM), Likn_, Likn32_);
     }
     Rotated own;
-    half_rotate_into(PsiT, own);
+    half_rotate_into(PsiT, own, true);
     PsiT_ = own.PsiT;
     Lnak_ = own.Lnak;
     haj_ = own.haj;
@@ -122,7 +122,10 @@ CholeskyOps::CholeskyOps(Context& c, int walker_type, int N, int nup, int ndown,
 // The half-rotated tensors of one determinant (RealDenseHamiltonian.cpp:141-163): per spin
 // block C[a][(k,m)] = sum_i PsiT[a][i] Likn[i][(k,m)], permuted to Lnak[m][a][k]; haj = PsiT h1
 // (half_rotate_hamiltonian, one_body.hpp); the real and FP32 copies the contractions read.
-void CholeskyOps::half_rotate_into(const z64* PsiT, Rotated& r) const {
+// own: the hamiltonian's own determinant, which vbias contracts and whose complex tensor callers
+// read (Lnak()).  A further real determinant of an expansion, of which there may be many, drops the
+// complex tensor once its real copies exist and has no operand of vbias.
+void CholeskyOps::half_rotate_into(const z64* PsiT, Rotated& r, bool own) const {
   hipStream_t s = ctx_.stream();
   const int N = N_, M = M_, nel_ = nel();
   try {
@@ -175,12 +178,17 @@ void CholeskyOps::half_rotate_into(const z64* PsiT, Rotated& r) const {
       if (r.real) {
         r.Lnak_r32 = dalloc<float>((size_t)M * nel_ * N);
         real_part_f32(s, (long)M * nel_ * N, r.Lnak, r.Lnak_r32);
-        build_split(r);
       } else {
         r.Lnak32 = dalloc<c32>((size_t)M * nel_ * N);
         cast_z64_c32(s, (long)M * nel_ * N, r.Lnak, r.Lnak32);
       }
     }
+    if (r.real && !own) {
+      AFQ_HIP(hipStreamSynchronize(s));
+      AFQ_HIP(hipFree(r.Lnak));
+      r.Lnak = nullptr;
+    }
+    if (prec_ == kMixed && r.real) build_split(r, own);
   } catch (...) {
     release(r);
     throw;
@@ -188,15 +196,16 @@ void CholeskyOps::half_rotate_into(const z64* PsiT, Rotated& r) const {
 }
 
 // The FP32 half-rotated tensor split into bfloat16 pieces (split3.hpp): per spin block packed by
-// rows (m) over (a, k) for vbias and by tiles of two vectors for the exchange.  A tensor that is not
-// finite or beyond the packed operands' 32-bit offsets keeps the FP32 products.
-void CholeskyOps::build_split(Rotated& r) const {
+// tiles of two vectors for the exchange and, for the hamiltonian's own determinant, by rows (m) over
+// (a, k) for vbias.  A tensor that is not finite or beyond the packed operands' 32-bit offsets keeps
+// the FP32 products.
+void CholeskyOps::build_split(Rotated& r, bool own) const {
   hipStream_t s = ctx_.stream();
   const int N = N_, M = M_, ns[2] = {nup_, ndown_};
   int* bad = scratch_as<int>(ctx_, "setup_bad", 1);
   AFQ_HIP(hipMemsetAsync(bad, 0, sizeof(int), s));
   r.s3_off[1] = s3::bytes_real(M, (long)nup_ * N);
-  if (s3::fits(M, (long)std::max(nup_, ndown_) * N, false))
+  if (own && s3::fits(M, (long)std::max(nup_, ndown_) * N, false))
     r.Lnak_s3 = dalloc<char>(r.s3_off[1] + s3::bytes_real(M, (long)ndown_ * N));
   for (int sp = 0; sp < 2; ++sp) {
     if (ns[sp] == 0) continue;
@@ -259,7 +268,7 @@ void CholeskyOps::build_pairs() {
 
 Rotated CholeskyOps::rotate(const z64* PsiT) const {
   Rotated r;
-  half_rotate_into(PsiT, r);
+  half_rotate_into(PsiT, r, false);
   AFQ_HIP(hipStreamSynchronize(ctx_.stream()));
   return r;
 }

@@ -128,14 +128,15 @@ void orthogonalize(Context& c, z64* Phi, long phi_bs, int W, int N, int n, z64* 
 // half_rotate_hamiltonian): device buffers owned by whoever built them.
 struct Rotated {
   z64* PsiT = nullptr;        // [nel][N]
-  z64* Lnak = nullptr;        // [M][nup][N], then [M][ndown][N] for COLLINEAR
+  z64* Lnak = nullptr;        // [M][nup][N], then [M][ndown][N] for COLLINEAR (null for a further
+                              // real determinant of an expansion)
   z64* haj = nullptr;         // [nel][N]
   double* Lnak_r = nullptr;   // its real part, when the determinant is real
   float* Lnak_r32 = nullptr;  // FP32 real part (mixed precision, real determinant)
   c32* Lnak32 = nullptr;      // FP32 copy (mixed precision, complex determinant)
   bool real = false;
-  // mixed precision, real determinant: Lnak_r32 split into bfloat16 pieces and packed for vbias
-  // (split3.hpp, one block per spin at s3_off); null when it does not apply
+  // mixed precision, the hamiltonian's own real determinant: Lnak_r32 split into bfloat16 pieces and
+  // packed for vbias (split3.hpp, one block per spin at s3_off); null when it does not apply
   char* Lnak_s3 = nullptr;
   size_t s3_off[2] = {0, 0};
   // and packed for the fused exchange (exchange.hip; electrons <= 40), one block per spin
@@ -241,12 +242,12 @@ class CholeskyOps {
   size_t s3_off_[2] = {0, 0};
   char* Lexx_s3_[2] = {nullptr, nullptr};
   void build_pairs();
-  // packs the FP32 half-rotated tensor for vbias and the exchange (split3.hpp)
-  void build_split(Rotated& r) const;
+  // packs the FP32 half-rotated tensor for the exchange and (own) vbias (split3.hpp)
+  void build_split(Rotated& r, bool own) const;
   void free_all();
   void exchange_spin(int sp, const z64* Gblk, int W, z64* part, z64* Kl, Precision prec,
                      const Rotated& t) const;
-  void half_rotate_into(const z64* PsiT, Rotated& r) const;
+  void half_rotate_into(const z64* PsiT, Rotated& r, bool own) const;
   static bool crg_path();
   // the force bias in FP32 from G in FP64 or already rounded to FP32
   template <typename TG>

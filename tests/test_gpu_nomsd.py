@@ -396,3 +396,29 @@ def test_nomsd_measurements_vs_oracle(gpu, closed):
     prop.close()
     trial.close()
     assert max(e1, e2, e3, e4) < TOL
+
+
+def test_memory_of_a_determinant(gpu):
+    """A further real determinant of a mixed-precision expansion keeps what its energy reads: the
+    half-rotated tensor in FP64, in FP32 and packed for the fused exchange.  That is 8 + 4 + 6 = 18
+    bytes a value where nothing is padded (n a multiple of 8, N of 32); five allocations a
+    determinant rounded up by at most 2 MiB each are another 1.7."""
+    afq, ctx, torch = gpu
+    from safire_amd.nomsd import NOMSD
+    N, n, M, ndet = 64, 24, 4000, 5
+    say(f"case: NOMSD memory N={N} n={n} M={M} ndet={ndet}")
+    p = make_problem(N, n, M, 41)
+    ham = afq.HamiltonianOperations(ctx, p.h1, p.Likn, p.PsiT, n, precision=afq.AFQ_MIXED)
+    rng = np.random.default_rng(3)
+    rows = [p.PsiT] + [np.linalg.qr(p.PsiT.real.T + 0.2 * rng.normal(size=(N, n)))[0].T
+                       for _ in range(ndet - 1)]
+    PsiT = afq.device_tensor(np.stack(rows), np.complex128)
+    NOMSD(ham, PsiT, np.ones(ndet)).close()  # (the set-up scratch exists from here on)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    trial = NOMSD(ham, PsiT, np.ones(ndet))
+    torch.cuda.synchronize()
+    per = (free - torch.cuda.mem_get_info()[0]) / ((ndet - 1) * M * n * N)
+    say(f"  {per:.2f} bytes a value")
+    trial.close()
+    assert per <= 20
