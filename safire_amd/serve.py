@@ -71,18 +71,44 @@ def poisson_jobs(n_jobs=200, rate=4.0, seed=2024, steps=400, lscale=0.1):
                     10_000 + i, steps=steps, lscale=lscale) for i in range(n_jobs)]
 
 
+def _packed(rows: int, K: int) -> int:
+    """Bytes of a real operand of the split products: three bfloat16 pieces a value, in blocks of 16
+    rows x 32 values."""
+    return -(-rows // 16) * -(-K // 32) * 3072
+
+
+def _packed_exchange(items: int, n: int, N: int) -> int:
+    """The same for the exchange kernel: items of n rows in tiles of two, n padded to a multiple of 8."""
+    return -(-items // 2) * -(-n // 8) * -(-N // 32) * 3072
+
+
+def resident_bytes(spec: JobSpec) -> int:
+    """What a mixed-precision hamiltonian with a real closed-shell trial holds: the Cholesky tensor
+    and the half-rotated tensor in FP64 (the latter complex and real), in FP32 and packed."""
+    N, n, M = spec.N, spec.nup, spec.M
+    pairs = N * (N + 1) // 2
+    packed = _packed(pairs, M) + 4 * pairs + _packed(M, n * N)
+    if n <= 40:
+        packed += _packed_exchange(M, n, N)
+    return N * N * M * 12 + M * n * N * 28 + N * N * 16 + n * N * 32 + packed
+
+
 def footprint(spec: JobSpec) -> int:
-    """Upper estimate of a job's device memory (bytes): resident tensors, walkers, step and
+    """Upper estimate of a job's device memory (bytes): resident tensors, walkers, set-up, step and
     energy scratch of a mixed-precision context."""
     N, n, M, W = spec.N, spec.nup, spec.M, spec.W
-    ham = N * N * M * 12 + M * n * N * (16 + 12 + 8) + n * N * M * 16 + N * N * 64
+    setup = n * N * M * 16 + N * N * 64
     walkers = W * N * n * 16 + W * 5 * 16
-    step = (W * n * N * 16 + W * M * 24 + W * N * N * 8 + 3 * W * N * n * 8
-            + 4 * W * n * n * 16 + W * N * n * 16)
+    step = (W * n * N * 24 + W * M * 24 + W * N * N * 8 + 3 * W * N * n * 8
+            + 6 * W * n * n * 16 + W * N * n * 32)
+    # the packed fields and density matrices, and vbias's K slices (16 at most)
+    step += 2 * _packed(W, M) + 2 * _packed(W, n * N) + min(16, max(1, n * N // 128)) * W * M * 8
+    # the FP64 energy that starts a job takes T by chunks of at most 1 GiB
     per_m = W * n * n * 16
-    mc = max(1, min(M, (1 << 30) // max(per_m, 1)))
-    energy = per_m * mc + W * M * 16 + W * n * N * 24 + W * 64
-    return int(1.15 * (ham + walkers + step + energy)) + (64 << 20)
+    energy = per_m * max(1, min(M, (1 << 30) // max(per_m, 1)))
+    energy += W * M * 16 + W * n * N * 16 + W * (M // 8 + 4) * 16
+    energy += 2 * _packed_exchange(W, n, N) if n <= 40 else W * n * N * 8
+    return int(1.15 * (resident_bytes(spec) + setup + walkers + step + energy)) + (64 << 20)
 
 
 class _Active:

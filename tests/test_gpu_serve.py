@@ -1,6 +1,8 @@
 """Serving loop: jobs of different sizes admitted while others run give the same result alone and
 in the mix (fixed per-job seeds, fixed-order reductions: bit-identical energies expected; the
 stated tolerance is 1e-12 relative)."""
+import dataclasses
+import gc
 import sys
 
 import numpy as np
@@ -63,6 +65,52 @@ def test_largest_serving_job_alone_equals_mix():
     assert alone.energy == m.energy
     for r in mixed.values():
         assert np.isfinite(r.energy) and not r.collapsed, r
+
+
+@pytest.mark.parametrize("N,W", [(32, 512), (160, 64), (160, 512)])
+def test_footprint_covers_the_job(N, W):
+    """footprint(): its resident part is at least what a mixed-precision hamiltonian holds and
+    not over it by more than a tenth (and the 2 MiB a separate allocation may round up to), and
+    the whole is at least what the job holds after steps and an energy evaluation."""
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from safire_amd import afq, serve
+    from safire_amd.synthetic import make_problem
+    spec = serve.JobSpec(0, 0.0, N, N // 4, 5 * N, W, 5, steps=6, equilibration=2,
+                         measure_interval=2)
+    say(f"case: footprint N={N} W={W}")
+    problem = make_problem(N, spec.nup, spec.M, 5, lscale=0.1)
+
+    def used(since):
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+        return since - torch.cuda.mem_get_info()[0]
+    # (code objects and the library's own fixed buffers are loaded by a first small job)
+    small = serve._Active(dataclasses.replace(spec, N=32, nup=8, M=160, W=64),
+                          make_problem(32, 8, 160, 5, lscale=0.1), afq.AFQ_MIXED, 0.0)
+    small.advance(6)
+    torch.cuda.synchronize()
+    del small
+    gc.collect()
+    ctx = afq.Context(0, stream=torch.cuda.Stream())
+    torch.cuda.empty_cache()
+    free = torch.cuda.mem_get_info()[0]
+    ham = afq.HamiltonianOperations(ctx, problem.h1, problem.Likn, problem.PsiT, spec.nup,
+                                    precision=afq.AFQ_MIXED)
+    held = used(free) - ctx.scratch_bytes()
+    say(f"  hamiltonian {held} bytes, estimated {serve.resident_bytes(spec)}")
+    assert held <= serve.resident_bytes(spec) + (16 << 20)
+    assert serve.resident_bytes(spec) <= 1.1 * held + (16 << 20)
+    del ham, ctx
+    gc.collect()
+    torch.cuda.empty_cache()
+    free = torch.cuda.mem_get_info()[0]
+    job = serve._Active(spec, problem, afq.AFQ_MIXED, 0.0)
+    job.advance(6)
+    total = used(free)
+    say(f"  job {total} bytes, estimated {serve.footprint(spec)}")
+    assert total <= serve.footprint(spec)
 
 
 def test_collapse_at_the_benchmark_amplitude_is_reported():
