@@ -355,6 +355,9 @@ void CholeskyOps::vHS(const void* X, int W, double dt, void* V, Precision prec) 
   const double a = std::sqrt(dt);
   const long NN = (long)N_ * N_;
   const size_t esz = prec == kFP64 ? sizeof(z64) : sizeof(c32);
+  char* A = nullptr;  // the packed fields of the split products
+  if (prec != kFP64 && Lpair_s3_ && crg_path() && s3::fits(W, M_, true))
+    A = static_cast<char*>(ctx_.scratch_kept("s3_X", s3::bytes_cplx(W, M_)));
   for (int l = 0; l < nl_; ++l) {
     // block l of V [nl][W][N][N] from block l of L
     char* Vl = reinterpret_cast<char*>(V) + (size_t)l * W * NN * esz;
@@ -383,11 +386,10 @@ void CholeskyOps::vHS(const void* X, int W, double dt, void* V, Precision prec) 
         AFQ_CHECK(prec_ == kMixed, kErrState, "FP32 tensors were not built (precision FP64)");
         gemm::EpiStoreSym<float, float> e{reinterpret_cast<c32*>(Vl), NN, 0, (float)a, 0.f, N_, nb};
         const c32* X32 = reinterpret_cast<const c32*>(X);
-        if (Lpair_s3_ && crg_path() && s3::fits(W, M_, true)) {
+        if (A) {
           // on the bfloat16 matrix cores over the N(N+1)/2 distinct pairs, k groups from the
           // last Cholesky vector to the first
           const int np = N_ * (N_ + 1) / 2;
-          char* A = scratch_as<char>(ctx_, "s3_A", s3::bytes_cplx(W, M_));
           if (l == 0) s3::pack_cplx(s, W, M_, X32, M_, A);
           s3::vhs_pairs(s, W, np, M_, A, Lpair_s3_ + l * s3::bytes_real(np, M_), pairs_, N_,
                         (float)a, reinterpret_cast<c32*>(Vl));
@@ -437,13 +439,15 @@ void CholeskyOps::vbias_f32(const cplx<TG>* G, int W, double dt, z64* v) const {
     size_t loff = sp == 0 ? 0 : (size_t)M_ * nup_ * N_;
     const long K = (long)ns * N_;
     EpiStore<float, double> e{v, M_, 0, a, 0.f, acc};
-    if (Lnak_s3_ && crg_path() && s3::fits(W, K, true)) {
+    char* Gp = nullptr;
+    if (Lnak_s3_ && crg_path() && s3::fits(W, K, true))
+      Gp = static_cast<char*>(ctx_.scratch_kept("s3_G", s3::bytes_cplx(W, K)));
+    if (Gp) {
       // on the bfloat16 matrix cores, K cut into slices so that the tiles fill the machine
-      char* A = scratch_as<char>(ctx_, "s3_A", s3::bytes_cplx(W, K));
-      s3::pack_cplx(s, W, (int)K, G + goff, (long)nel_ * N_, A);
+      s3::pack_cplx(s, W, (int)K, G + goff, (long)nel_ * N_, Gp);
       const s3::Plan p = s3::plan(W, M_, (int)s3::k_groups(K), true);
       c32* ws = p.ksplit > 1 ? scratch_as<c32>(ctx_, "s3_ws", (size_t)p.ksplit * W * M_) : nullptr;
-      s3::vbias(s, W, M_, (int)K, A, Lnak_s3_ + s3_off_[sp], p, a, acc != 0, v, ws);
+      s3::vbias(s, W, M_, (int)K, Gp, Lnak_s3_ + s3_off_[sp], p, a, acc != 0, v, ws);
       continue;
     }
     constexpr bool g32 = sizeof(TG) == 4;
@@ -516,7 +520,7 @@ void CholeskyOps::exchange_spin(int sp, const z64* Gblk, int W, z64* part, z64* 
     const int nparts = exx_fused_parts(M_);
     const size_t per2 = s3::bytes_exx_G(2, ns, N_);
     const int run = 2 * (int)std::max<size_t>(1, (size_t)0x7FFF0000u / per2);
-    char* Gp = scratch_as<char>(ctx_, "s3_A", s3::bytes_exx_G(std::min(W, run), ns, N_));
+    char* Gp = scratch_as<char>(ctx_, "en_Gp", s3::bytes_exx_G(std::min(W, run), ns, N_));
     for (int w = 0; w < W; w += run) {
       const int wc = std::min(run, W - w);
       s3::pack_exx_G(s, wc, ns, N_, Gblk + (size_t)w * ns * N_, Gp);

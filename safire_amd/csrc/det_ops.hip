@@ -35,6 +35,7 @@ Context::~Context() {
   (void)hipStreamSynchronize(stream_);
   for (auto& kv : bufs_)
     if (kv.second.p) (void)hipFree(kv.second.p);
+  for (auto& b : kept_) (void)hipFree(b.p);
   if (own_stream_) (void)hipStreamDestroy(stream_);
 }
 
@@ -68,8 +69,26 @@ void* Context::scratch(const std::string& name, size_t bytes) {
   return b.p;
 }
 
+void* Context::scratch_kept(const std::string& name, size_t bytes) {
+  auto it = bufs_.find(name);
+  const Buf old = it == bufs_.end() ? Buf{} : it->second;
+  if (old.p && old.bytes < bytes) {
+    if (no_alloc_ || capturing()) return nullptr;
+    kept_.push_back(old);
+    bufs_.erase(it);
+    try {
+      return scratch(name, std::max(bytes, 2 * old.bytes));
+    } catch (const Error&) {  // no room for twice the size
+      return scratch(name, bytes);
+    }
+  }
+  if (!old.p && (no_alloc_ || capturing())) return nullptr;
+  return scratch(name, bytes);
+}
+
 size_t Context::scratch_bytes() const {
   size_t t = 0;
+  for (auto& b : kept_) t += b.bytes;
   for (auto& kv : bufs_) t += kv.second.bytes;
   return t;
 }

@@ -29,6 +29,10 @@ class Context {
   hipStream_t stream() const { return stream_; }
   // Scratch buffer `name` of at least `bytes`; contents are not preserved across growth.
   void* scratch(const std::string& name, size_t bytes);
+  // As scratch(), but a buffer that grows is kept until the context ends (its successor has at least
+  // twice its size), so a graph captured by the caller never holds a freed address; null instead of
+  // an error where the buffer would have to grow inside a capture or an allocation-free call.
+  void* scratch_kept(const std::string& name, size_t bytes);
   size_t scratch_bytes() const;
   bool capturing() const;
   // Incremented whenever a scratch buffer is freed to grow it: a HIP graph captured under an
@@ -49,6 +53,7 @@ class Context {
     size_t bytes = 0;
   };
   std::map<std::string, Buf> bufs_;
+  std::vector<Buf> kept_;  // outgrown buffers of scratch_kept
   uint64_t gen_ = 0;
 };
 

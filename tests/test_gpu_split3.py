@@ -154,3 +154,46 @@ def test_tensors_outside_the_split_keep_the_fp32_product(gpu):
     assert not np.any(np.isfinite(V[:, 2, 4])) and not np.any(np.isfinite(V[:, 4, 2]))
     V[:, 2, 4] = V[:, 4, 2] = 0
     assert np.all(np.isfinite(V))
+
+
+@pytest.mark.parametrize("which", ["vHS", "vbias"])
+def test_captured_without_a_first_call(gpu, which):
+    """The first vHS or vbias of a context inside a HIP graph capture is recorded (a capture cannot
+    allocate: it takes the FP32 engine), and a graph that was captured after a first call keeps
+    giving its result when later calls with more walkers have made the workspace grow."""
+    afq, _, torch = gpu
+    N, n, M, W = 24, 5, 30, 8
+    print(f"case: captured {which}", flush=True)
+    p = make_problem(N, n, M, 8)
+    rng = np.random.default_rng(2)
+
+    def inputs(w):
+        s = (w, M) if which == "vHS" else (w, n, N)
+        x = afq.device_tensor(rng.normal(size=s) + 1j * rng.normal(size=s))
+        if which == "vHS":
+            return x.to(torch.complex64), afq.empty((w, N, N), torch.complex64)
+        return x, afq.empty((w, M), torch.complex128)
+
+    for warm in (False, True):
+        ctx = afq.Context(0)
+        ham = afq.HamiltonianOperations(ctx, p.h1, p.Likn, p.PsiT, n, precision=afq.AFQ_MIXED)
+        x, out = inputs(W)
+        if warm:
+            getattr(ham, which)(x, out, 0.01)
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=ctx.stream):
+            getattr(ham, which)(x, out, 0.01)
+        for grow in (1, 5, 40):
+            y, big = inputs(W * grow)
+            getattr(ham, which)(y, big, 0.01)
+            eager = torch.empty_like(out)
+            getattr(ham, which)(x, eager, 0.01)
+            out.zero_()
+            g.replay()
+            torch.cuda.synchronize()
+            a, b = afq.host(out), afq.host(eager)
+            if warm:
+                assert np.array_equal(a, b)
+            else:  # other kernels: 30 or 120 FP32 products of N(0, 1) numbers
+                assert np.max(np.abs(a - b)) < 1e-5 * np.max(np.abs(b))
