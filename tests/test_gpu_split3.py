@@ -156,6 +156,44 @@ def test_tensors_outside_the_split_keep_the_fp32_product(gpu):
     assert np.all(np.isfinite(V))
 
 
+# one K slice and several; both parts, one walker past FP32's range
+@pytest.mark.parametrize("N,n,nd,M,W", [(12, 3, 0, 40, 21), (33, 8, 0, 165, 40), (40, 9, 7, 96, 21)])
+def test_vbias_infinities_and_nan(gpu, N, n, nd, M, W):
+    """As test_infinities_and_nan for a density matrix."""
+    afq, ctx, torch = gpu
+    print(f"case: split vbias with infinities N={N} n={n}+{nd} M={M} W={W}", flush=True)
+    p = make_problem(N, n, M, 5)
+    ham = afq.HamiltonianOperations(
+        ctx, p.h1, p.Likn, np.concatenate([p.PsiT, p.PsiT[:nd]]), n, nd,
+        walker_type=afq.AFQ_COLLINEAR if nd else afq.AFQ_CLOSED, precision=afq.AFQ_MIXED)
+    rng = np.random.default_rng(1)
+    G = rng.normal(size=(W, n + nd, N)) + 1j * rng.normal(size=(W, n + nd, N))
+
+    def vbias(g):
+        v = afq.empty((W, M), torch.complex128)
+        ham.vbias(afq.device_tensor(g), v, 1.0)
+        return afq.host(v)
+    clean = vbias(G)
+    H = G.copy()
+    H[3, n - 1, 7] = np.inf
+    H[16, 0, N - 1] = complex(0.5, -1e39)
+    H[18, n + nd - 1, 0] = np.nan
+    H[20, 0, 0], H[20, n + nd - 1, N - 1] = np.inf, -np.inf
+    got = vbias(H)
+    os.environ["AFQ_CRGEMM"] = "0"
+    try:
+        ref = vbias(H)
+    finally:
+        del os.environ["AFQ_CRGEMM"]
+    rest = [w for w in range(W) if w not in (3, 16, 18, 20)]
+    assert np.array_equal(got[rest], clean[rest])
+    for part in (np.real, np.imag):
+        g, r = part(got), part(ref)
+        assert np.array_equal(np.isnan(g), np.isnan(r))
+        inf = np.isinf(r)
+        assert np.array_equal(np.isinf(g), inf) and np.array_equal(g[inf], r[inf])
+
+
 @pytest.mark.parametrize("which", ["vHS", "vbias"])
 def test_captured_without_a_first_call(gpu, which):
     """The first vHS or vbias of a context inside a HIP graph capture is recorded (a capture cannot
