@@ -37,19 +37,137 @@ using s3::bf16x8;
 constexpr int kXTiles = 2;  // tiles (pairs of wavefronts) per workgroup
 constexpr int kXVpw = 4;    // tiles a pair of wavefronts takes one after the other
 
+// LDS pitch of a column of T: the rows of both walkers plus 8, which keeps the 8 x 8 lane blocks of the
+// exchange reads on distinct banks
+template <int NB>
+constexpr int kXPitch = 16 * NB + 8;
+
+// What a wavefront of a tile works on
+struct XTile {
+  int W, ns, M, pair, cpart, lane;
+  float* tre;  // LDS: real parts of the vector's columns of T, then the imaginary parts
+  z64* Kl;
+};
+
+// Adds the exchange and Coulomb terms of vector 2 mt0 + mj, whose T lies in LDS.  A trace that is not
+// finite is left out and noted in bit 2 vp + mj of `left`; LAST adds just those.
+template <int NB, bool LAST>
+__device__ inline void exx_terms(const XTile& x, int vp, int mt0, int mj, double& xr, double& xi,
+                                 uint32_t& left) {
+  constexpr int NSP = 8 * NB, LDC = kXPitch<NB>;
+  const int xb = x.lane & 7, xa = x.lane >> 3;
+  const int m = 2 * mt0 + mj, w = 2 * x.pair + x.cpart;
+  if (m >= x.M || w >= x.W) return;  // uniform per wavefront
+  const float* ur = x.tre + x.cpart * NSP;
+  const float* ui = ur + NSP * LDC;
+  // exchange: sum_ab T_ab T_ba over 8 x 8 blocks (ib, ia) of (b, a), lane (xb, xa) taking
+  // b = 8 ib + xb, a = 8 ia + xa; the sum is symmetric in (a, b), so the blocks above the
+  // diagonal count twice and those below are skipped
+#pragma unroll
+  for (int ib = 0; ib < NB; ++ib)
+#pragma unroll
+    for (int ia = ib; ia < NB; ++ia) {
+      const int b = 8 * ib + xb, a = 8 * ia + xa;
+      const double pr = ur[a * LDC + b], pi = ui[a * LDC + b];  // T_ba
+      const double qr = ur[b * LDC + a], qi = ui[b * LDC + a];  // T_ab
+      const double wgt = (b < x.ns && a < x.ns) ? (ia == ib ? 1.0 : 2.0) : 0.0;
+      xr += wgt * (pr * qr - pi * qi);
+      xi += wgt * (pr * qi + pi * qr);
+    }
+  // Coulomb trace of this (walker, vector)
+  if (x.Kl) {
+    double kr = 0.0, ki = 0.0;
+    if (x.lane < x.ns) {
+      kr = ur[x.lane * LDC + x.lane];
+      ki = ui[x.lane * LDC + x.lane];
+    }
+    kr = wave_sum(kr);
+    ki = wave_sum(ki);
+    const bool fin = __builtin_isfinite(kr) && __builtin_isfinite(ki);  // the same in every lane
+    if (!LAST && !fin) left |= 1u << (2 * vp + mj);
+    if (x.lane == 0 && (LAST ? (left >> (2 * vp + mj) & 1u) != 0 : fin)) {
+      z64* o = x.Kl + (long)w * x.M + m;
+      *o = z64{o->re + kr, o->im + ki};
+    }
+  }
+}
+
+// The sums again for walkers whose T holds an infinity or NaN, with T from plain FP32 products: the split
+// products turn an infinity into NaN (split3.hpp).  A walker with a NaN in both parts of G is NaN
+// throughout either way.  One 16 x 16 block at a time: its registers must not weigh on the kernel's
+// loop.  The energy of 1024 walkers (N = 200, n = 40, M = 1600) takes 10.4 ms, with 1 and 100 infinite
+// ones 11.1 and 26.8, with NaN ones 10.5.
+template <int NB>
+__device__ inline z64 exx_redo(const XTile& x, int KG, const char* G, uint32_t gbytes,
+                               const char* L, uint32_t lbytes, int tile, int mtile0, uint32_t* flags,
+                               bool redo, z64 sum, uint32_t left) {
+  constexpr int NSP = 8 * NB, LDC = kXPitch<NB>;
+  const int l16 = x.lane * 16, fr = x.lane & 15, fk = x.lane >> 4;
+  const auto rG = s3::resource(G, gbytes);
+  const auto rL = s3::resource(L, lbytes);
+  const uint32_t oa = (uint32_t)(((long)x.pair * 2 + x.cpart) * NB * KG * s3::kBlock);
+  // the walkers with a NaN in this wavefront's part of G
+  uint32_t nan = 0;
+#pragma unroll 1
+  for (int i = 0; i < NB; ++i)
+    for (int g = 0; g < KG; ++g) {
+      const bf16x8 p = s3::load_block<0>(rG, oa + (uint32_t)((i * KG + g) * (int)s3::kBlock), l16);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) nan |= p[e] != p[e] ? (16 * i + fr < NSP ? 1u : 2u) : 0u;
+    }
+  const bool n0 = __ballot(nan & 1u) != 0, n1 = __ballot(nan & 2u) != 0;
+  if (x.lane == 0) flags[2 * tile + x.cpart] = (n0 ? 1u : 0u) | (n1 ? 2u : 0u);
+  __syncthreads();
+  redo = redo && !((flags[2 * tile] & flags[2 * tile + 1]) >> x.cpart & 1u);
+  __syncthreads();
+  if (x.lane == 0) flags[2 * tile + x.cpart] = redo;
+  __syncthreads();
+  bool any = false;
+#pragma unroll
+  for (int i = 0; i < 2 * kXTiles; ++i) any = any || flags[i];
+  if (__ballot(any) == 0) return sum;  // uniform per workgroup
+  const bool own = __ballot(flags[2 * tile] || flags[2 * tile + 1]) != 0;
+  double xr = 0.0, xi = 0.0;
+  float* tmine = x.tre + (x.cpart ? NSP * LDC : 0);
+#pragma unroll 1
+  for (int v = 0; v < 2 * kXVpw; ++v) {
+    const int mt0 = mtile0 + v / 2, mj = v & 1;
+    __syncthreads();
+#pragma unroll 1
+    for (int ij = 0; ij < NB * NB && own && 2 * mt0 < x.M; ++ij) {
+      const int i = ij / NB, j = ij % NB, col = 16 * j + fr - mj * NSP;
+      const uint32_t ob = (uint32_t)(((long)mt0 * NB + j) * KG * s3::kBlock);
+      f32x4 c = {0.f, 0.f, 0.f, 0.f};
+      for (int g = 0; g < KG; ++g) {
+        float a[8], b[8];
+        s3::load_sums(a, rG, oa + (uint32_t)((i * KG + g) * (int)s3::kBlock), l16);
+        s3::load_sums(b, rL, ob + (uint32_t)(g * (int)s3::kBlock), l16);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) c = s3::mfma_f32(a[e], b[e], c);
+      }
+      if (col < 0 || col >= NSP) continue;
+      // (an infinity times the zeros that pad a vector to NSP rows is NaN)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if ((16 * i + 4 * fk + r) % NSP >= x.ns || col >= x.ns) c[r] = 0.f;
+      *reinterpret_cast<f32x4*>(tmine + col * LDC + 16 * i + 4 * fk) = c;
+    }
+    __syncthreads();
+    exx_terms<NB, true>(x, v / 2, mt0, mj, xr, xi, left);
+  }
+  return redo ? z64{xr, xi} : sum;
+}
+
 template <int NB>
 __global__ void __launch_bounds__(128 * kXTiles, 2)
     k_exx_split(int W, int ns, int KG, int M, const char* __restrict__ G, uint32_t gbytes,
                 const char* __restrict__ L, uint32_t lbytes, int npairs, z64* __restrict__ part,
                 int nparts, z64* __restrict__ Kl) {
-  // LDS pitch of a column of T: the rows of both walkers plus 8, which keeps the 8 x 8 lane
-  // blocks of the exchange reads on distinct banks
-  constexpr int NSP = 8 * NB, R = 2 * NSP, LDC = R + 8;
+  constexpr int NSP = 8 * NB, LDC = kXPitch<NB>;
   extern __shared__ __align__(16) float smem_x[];  // [kXTiles][2][NSP * LDC]
+  __shared__ uint32_t flags[2 * kXTiles];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int cpart = wave & 1, tile = wave >> 1;  // real (0) or imaginary (1) part; the tile
-  const int fr = lane & 15, fk = lane >> 4;
-  const int xb = lane & 7, xa = lane >> 3;
   const long total = gridDim.x, xcd = blockIdx.x % 8, slot = blockIdx.x / 8;
   const long q = xcd * (total / 8) + min(xcd, total % 8) + slot;
   const int pair = (int)(q % npairs), chunk = (int)(q / npairs);
@@ -60,7 +178,9 @@ __global__ void __launch_bounds__(128 * kXTiles, 2)
   float* tre = smem_x + tile * 2 * NSP * LDC;
   float* tim = tre + NSP * LDC;
   float* tmine = cpart ? tim : tre;
+  XTile x{W, ns, M, pair, cpart, lane, tre, Kl};
   double xr = 0.0, xi = 0.0;  // exchange of walker 2 pair + cpart
+  uint32_t left = 0;          // bit 2 vp + mj: that vector's trace is left out
 
   for (int vp = 0; vp < kXVpw; ++vp) {
     const int mt0 = (chunk * kXTiles + tile) * kXVpw + vp;
@@ -117,6 +237,10 @@ __global__ void __launch_bounds__(128 * kXTiles, 2)
 #undef AFQ_LD
 #undef AFQ_MM
     }
+    // (opaque to the compiler, which would keep the reduction's LDS addresses in registers through the
+    // products and spill them: 60 bytes a lane and 1.8 % of the time at n = 40)
+    asm volatile("" : "+v"(x.lane));
+    const int fr = x.lane & 15, fk = x.lane >> 4;
     // one Cholesky vector (tile columns mj NSP .. mj NSP + NSP - 1) at a time through LDS,
     // column-major: T[row][c] at c LDC + row, so each lane stores its four accumulator rows as
     // one 16-byte write
@@ -132,39 +256,21 @@ __global__ void __launch_bounds__(128 * kXTiles, 2)
           *reinterpret_cast<f32x4*>(tmine + col * LDC + 16 * i + 4 * fk) = c[i][j];
       }
       __syncthreads();
-      const int m = 2 * mt0 + mj, w = 2 * pair + cpart;
-      if (m >= M || w >= W) continue;  // uniform per wavefront; the barriers are above
-      const float* ur = tre + cpart * NSP;
-      const float* ui = tim + cpart * NSP;
-      // exchange: sum_ab T_ab T_ba over 8 x 8 blocks (ib, ia) of (b, a), lane (xb, xa) taking
-      // b = 8 ib + xb, a = 8 ia + xa; the sum is symmetric in (a, b), so the blocks above the
-      // diagonal count twice and those below are skipped
-#pragma unroll
-      for (int ib = 0; ib < NB; ++ib)
-#pragma unroll
-        for (int ia = ib; ia < NB; ++ia) {
-          const int b = 8 * ib + xb, a = 8 * ia + xa;
-          const double pr = ur[a * LDC + b], pi = ui[a * LDC + b];  // T_ba
-          const double qr = ur[b * LDC + a], qi = ui[b * LDC + a];  // T_ab
-          const double wgt = (b < ns && a < ns) ? (ia == ib ? 1.0 : 2.0) : 0.0;
-          xr += wgt * (pr * qr - pi * qi);
-          xi += wgt * (pr * qi + pi * qr);
-        }
-      // Coulomb trace of this (walker, vector)
-      if (Kl) {
-        double kr = 0.0, ki = 0.0;
-        if (lane < ns) {
-          kr = ur[lane * LDC + lane];
-          ki = ui[lane * LDC + lane];
-        }
-        kr = wave_sum(kr);
-        ki = wave_sum(ki);
-        if (lane == 0) {
-          z64* o = Kl + (long)w * M + m;
-          *o = z64{o->re + kr, o->im + ki};
-        }
-      }
+      exx_terms<NB, false>(x, vp, mt0, mj, xr, xi, left);
     }
+  }
+  const bool redo = __ballot(!(__builtin_isfinite(xr) && __builtin_isfinite(xi))) != 0;
+  if (lane == 0) flags[wave] = redo;
+  __syncthreads();
+  bool any = false;
+#pragma unroll
+  for (int i = 0; i < 2 * kXTiles; ++i) any = any || flags[i];
+  if (__ballot(any) != 0) {  // uniform per workgroup
+    __syncthreads();  // (the flags are read)
+    const z64 r = exx_redo<NB>(x, KG, G, gbytes, L, lbytes, tile,
+                               (chunk * kXTiles + tile) * kXVpw, flags, redo, z64{xr, xi}, left);
+    xr = r.re;
+    xi = r.im;
   }
   const double er = wave_sum(xr), ei = wave_sum(xi);
   const int w = 2 * pair + cpart;

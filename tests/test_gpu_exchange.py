@@ -132,3 +132,46 @@ def test_fused_exchange_collinear_coulomb_vectors(gpu):
     e = afq.empty((W, 3), torch.complex128)
     ham.energy_spin(1, e, afq.device_tensor(Gb), None, addEJ=False, precision=afq.AFQ_FP64)
     assert per_walker(afq.host(e)[:, 1], -0.5 * np.einsum("wmba,wmab->w", T, T)) < 1e-10
+
+
+@pytest.mark.parametrize("N,n,M,W", [(24, 8, 33, 7), (20, 5, 17, 6), (9, 1, 3, 5), (70, 40, 9, 6)])
+def test_infinite_density(gpu, N, n, M, W):
+    """Walkers whose G holds an infinity, a value past FP32's range or a NaN: the exchange, the
+    Coulomb energy and the Coulomb vectors are infinite or NaN where the sums over the products
+    G L (real and imaginary parts each of their own) are, and the other walkers keep their bits."""
+    afq, torch = gpu
+    say(f"case: fused exchange with infinities N={N} n={n} M={M} W={W}")
+    p = make_problem(N, n, M, seed=77)
+    ctx = afq.Context(0)
+    ham = afq.HamiltonianOperations(ctx, p.h1, p.Likn, p.PsiT, n, precision=afq.AFQ_MIXED)
+    G, _ = orc.mixed_density_matrix(p.PsiT, random_walkers(p, W, seed=5))
+
+    def evaluate(g):
+        e = afq.empty((W, 3), torch.complex128)
+        k = afq.empty((W, M), torch.complex128)
+        ham.energy_spin(0, e, afq.device_tensor(g), k, precision=afq.AFQ_MIXED)
+        return afq.host(e)[:, 1:], afq.host(k)
+    clean = evaluate(G)
+    H = G.copy()
+    H[0, 0, 3] = complex(np.inf, 0.25)
+    H[2, n - 1, N - 1] = complex(0.5, -1e39)
+    H[3, n // 2, 0] = complex(np.nan, 1.0)
+    H[4, 0, 1], H[4, 0, 2] = np.inf, complex(0.0, np.inf)
+    got = evaluate(H)
+    L = ham.tensors()[0].real.reshape(M, n, N).astype(np.float32).astype(np.float64)
+    with np.errstate(all="ignore"):
+        g32 = H.astype(np.complex64)
+        tr, ti = (np.einsum("wbk,mak->wmba", x.astype(np.float64), L) for x in (g32.real, g32.imag))
+        ur, ui = tr.transpose(0, 1, 3, 2), ti.transpose(0, 1, 3, 2)
+        kr, ki = (np.trace(x, axis1=2, axis2=3) for x in (tr, ti))
+        sums = [(x.reshape(W, -1).sum(1), y.reshape(W, -1).sum(1)) for x, y in
+                ((-(tr * ur - ti * ui), -(tr * ui + ti * ur)), (kr * kr - ki * ki, 2 * kr * ki))]
+    ref = [tuple(np.stack([s[part] for s in sums], axis=1) for part in (0, 1)), (kr, ki)]
+    rest = [w for w in range(W) if w not in (0, 2, 3, 4)]
+    for g, r, c in zip(got, ref, clean):
+        assert np.array_equal(g[rest], c[rest])
+        for x, y in zip((g.real, g.imag), r):
+            assert np.array_equal(np.isnan(x), np.isnan(y))
+            inf = np.isinf(y)
+            assert np.array_equal(np.isinf(x), inf) and np.array_equal(x[inf], y[inf])
+    assert np.isinf(kr).any()
