@@ -197,8 +197,9 @@ void CholeskyOps::half_rotate_into(const z64* PsiT, Rotated& r, bool own) const 
 
 // The FP32 half-rotated tensor split into bfloat16 pieces (split3.hpp): per spin block packed by
 // tiles of two vectors for the exchange and, for the hamiltonian's own determinant, by rows (m) over
-// (a, k) for vbias.  A tensor that is not finite or beyond the packed operands' 32-bit offsets keeps
-// the FP32 products.
+// (a, k) for vbias.  A tensor that is not finite keeps the FP32 products, as does vbias beyond the
+// packed operand's 32-bit offsets and the exchange from 4 GiB in FP32 (its packed form, half as large
+// again and padded, is taken in runs).
 void CholeskyOps::build_split(Rotated& r, bool own) const {
   hipStream_t s = ctx_.stream();
   const int N = N_, M = M_, ns[2] = {nup_, ndown_};
@@ -212,9 +213,8 @@ void CholeskyOps::build_split(Rotated& r, bool own) const {
     const float* L = r.Lnak_r32 + (sp == 0 ? 0 : (size_t)M * nup_ * N);
     if (r.Lnak_s3)
       s3::pack_rows(s, M, ns[sp] * N, L, (long)ns[sp] * N, r.Lnak_s3 + r.s3_off[sp], bad);
-    const size_t eb = s3::bytes_exx_L(M, ns[sp], N);
-    if (std::max(nup_, ndown_) <= 40 && eb < (size_t)0xFFFF0000u) {
-      r.Lexx_s3[sp] = dalloc<char>(eb);
+    if (std::max(nup_, ndown_) <= 40 && (size_t)M * ns[sp] * N * sizeof(float) < (1UL << 32)) {
+      r.Lexx_s3[sp] = dalloc<char>(s3::bytes_exx_L(M, ns[sp], N));
       s3::pack_exx_L(s, M, ns[sp], N, L, r.Lexx_s3[sp], bad);
     }
   }

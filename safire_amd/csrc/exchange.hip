@@ -24,6 +24,8 @@
 // 4 VPW Cholesky vectors; workgroups are renumbered so that each XCD processes a contiguous run
 // with the walker pair fastest, so the workgroups resident on one XCD share their Cholesky vectors
 // through its L2.
+#include <algorithm>
+
 #include "ops.hpp"
 #include "split3.hpp"
 
@@ -44,7 +46,7 @@ constexpr int kXPitch = 16 * NB + 8;
 
 // What a wavefront of a tile works on
 struct XTile {
-  int W, ns, M, pair, cpart, lane;
+  int W, ns, M, ldk, pair, cpart, lane;
   float* tre;  // LDS: real parts of the vector's columns of T, then the imaginary parts
   z64* Kl;
 };
@@ -86,7 +88,7 @@ __device__ inline void exx_terms(const XTile& x, int vp, int mt0, int mj, double
     const bool fin = __builtin_isfinite(kr) && __builtin_isfinite(ki);  // the same in every lane
     if (!LAST && !fin) left |= 1u << (2 * vp + mj);
     if (x.lane == 0 && (LAST ? (left >> (2 * vp + mj) & 1u) != 0 : fin)) {
-      z64* o = x.Kl + (long)w * x.M + m;
+      z64* o = x.Kl + (long)w * x.ldk + m;
       *o = z64{o->re + kr, o->im + ki};
     }
   }
@@ -160,7 +162,7 @@ __device__ inline z64 exx_redo(const XTile& x, int KG, const char* G, uint32_t g
 
 template <int NB>
 __global__ void __launch_bounds__(128 * kXTiles, 2)
-    k_exx_split(int W, int ns, int KG, int M, const char* __restrict__ G, uint32_t gbytes,
+    k_exx_split(int W, int ns, int KG, int M, int ldk, const char* __restrict__ G, uint32_t gbytes,
                 const char* __restrict__ L, uint32_t lbytes, int npairs, z64* __restrict__ part,
                 int nparts, z64* __restrict__ Kl) {
   constexpr int NSP = 8 * NB, LDC = kXPitch<NB>;
@@ -178,7 +180,7 @@ __global__ void __launch_bounds__(128 * kXTiles, 2)
   float* tre = smem_x + tile * 2 * NSP * LDC;
   float* tim = tre + NSP * LDC;
   float* tmine = cpart ? tim : tre;
-  XTile x{W, ns, M, pair, cpart, lane, tre, Kl};
+  XTile x{W, ns, M, ldk, pair, cpart, lane, tre, Kl};
   double xr = 0.0, xi = 0.0;  // exchange of walker 2 pair + cpart
   uint32_t left = 0;          // bit 2 vp + mj: that vector's trace is left out
 
@@ -277,21 +279,28 @@ __global__ void __launch_bounds__(128 * kXTiles, 2)
   if (lane == 0 && w < W) part[(long)w * nparts + chunk * kXTiles + tile] = z64{er, ei};
 }
 
+// The Cholesky vectors in runs whose packed pieces the kernel's 32-bit offsets reach
 template <int NB>
 void launch_exx(hipStream_t s, int W, int ns, int N, int M, const char* G, const char* L,
                 z64* part, int nparts, z64* Kl) {
+  constexpr int kChunk = 2 * kXTiles * kXVpw;  // vectors of a workgroup
   const int npairs = ceil_div(W, 2);
-  const int nchunk = ceil_div(M, 2 * kXTiles * kXVpw);
-  AFQ_CHECK(nparts == nchunk * kXTiles, kErrArg, "exchange partial count");
-  const long blocks = (long)npairs * nchunk;
-  AFQ_CHECK(blocks < (1L << 31), kErrShape, "grid too large");
+  AFQ_CHECK(nparts == ceil_div(M, kChunk) * kXTiles, kErrArg, "exchange partial count");
   constexpr int NSP = 8 * NB;
-  constexpr size_t lds = sizeof(float) * kXTiles * 2 * NSP * (2 * NSP + 8);
+  constexpr size_t lds = sizeof(float) * kXTiles * 2 * NSP * kXPitch<NB>;
   static_assert(lds <= 64 * 1024, "the default LDS limit");
-  hipLaunchKernelGGL((k_exx_split<NB>), dim3((unsigned)blocks), dim3(128 * kXTiles), lds, s, W, ns,
-                     (int)s3::k_groups(N), M, G, (uint32_t)s3::bytes_exx_G(W, ns, N), L,
-                     (uint32_t)s3::bytes_exx_L(M, ns, N), npairs, part, nparts, Kl);
-  AFQ_LAUNCH_CHECK();
+  const size_t per = s3::bytes_exx_L(kChunk, ns, N);
+  const int run = (int)std::min<size_t>((size_t)M, kChunk * std::max<size_t>(1, 0xFFFF0000u / per));
+  for (int m0 = 0; m0 < M; m0 += run) {
+    const int mc = std::min(run, M - m0), c0 = m0 / kChunk;
+    const long blocks = (long)npairs * ceil_div(mc, kChunk);
+    AFQ_CHECK(blocks < (1L << 31), kErrShape, "grid too large");
+    hipLaunchKernelGGL((k_exx_split<NB>), dim3((unsigned)blocks), dim3(128 * kXTiles), lds, s, W,
+                       ns, (int)s3::k_groups(N), mc, M, G, (uint32_t)s3::bytes_exx_G(W, ns, N),
+                       L + c0 * per, (uint32_t)s3::bytes_exx_L(mc, ns, N), npairs,
+                       part + c0 * kXTiles, nparts, Kl ? Kl + m0 : nullptr);
+    AFQ_LAUNCH_CHECK();
+  }
 }
 
 }  // namespace
@@ -300,9 +309,8 @@ int exx_fused_parts(int M) { return ceil_div(M, 2 * kXTiles * kXVpw) * kXTiles; 
 
 void exchange_fused(hipStream_t s, int W, int ns, int N, int M, const void* G, const void* L,
                     z64* part, int nparts, z64* Kl) {
-  AFQ_CHECK(ns >= 1 && ns <= 40 && s3::bytes_exx_G(W, ns, N) < (size_t)0xFFFF0000u &&
-                s3::bytes_exx_L(M, ns, N) < (size_t)0xFFFF0000u,
-            kErrShape, "fused exchange supports 1 <= n <= 40 and packed operands under 4 GiB");
+  AFQ_CHECK(ns >= 1 && ns <= 40 && s3::bytes_exx_G(W, ns, N) < (size_t)0xFFFF0000u, kErrShape,
+            "fused exchange supports 1 <= n <= 40 and a packed G under 4 GiB");
   const char* g = static_cast<const char*>(G);
   const char* l = static_cast<const char*>(L);
   switch (s3::exx_nb(ns)) {

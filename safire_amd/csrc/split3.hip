@@ -50,7 +50,7 @@ void pack_cplx_t(hipStream_t s, long blocks, int K, const cplx<TIn>* X, long ld,
                  int nb, void* out) {
   const long KG = k_groups(K), waves = blocks * KG;
   if (waves == 0) return;
-  AFQ_CHECK(ceil_div(waves, 4) > 0, kErrShape, "grid too large");
+  AFQ_CHECK((waves + 3) / 4 < (1L << 31), kErrShape, "grid too large");
   hipLaunchKernelGGL((k_pack_cplx<TIn, ROWS>), dim3((unsigned)ceil_div(waves, 4)), dim3(256), 0, s,
                      blocks, K, (int)KG, X, ld, rmap, nb, static_cast<char*>(out));
   AFQ_LAUNCH_CHECK();
@@ -61,7 +61,7 @@ void pack_real_t(hipStream_t s, long blocks, int K, const float* X, long ld, con
                  void* out, int* bad) {
   const long KG = k_groups(K), waves = blocks * KG;
   if (waves == 0) return;
-  AFQ_CHECK(ceil_div(waves, 4) > 0, kErrShape, "grid too large");
+  AFQ_CHECK((waves + 3) / 4 < (1L << 31), kErrShape, "grid too large");
   hipLaunchKernelGGL((k_pack_real<ROWS>), dim3((unsigned)ceil_div(waves, 4)), dim3(256), 0, s,
                      blocks, K, (int)KG, X, ld, rmap, static_cast<char*>(out), bad);
   AFQ_LAUNCH_CHECK();

@@ -175,3 +175,47 @@ def test_infinite_density(gpu, N, n, M, W):
             inf = np.isinf(y)
             assert np.array_equal(np.isinf(x), inf) and np.array_equal(x[inf], y[inf])
     assert np.isinf(kr).any()
+
+
+def test_packed_tensor_past_4_gib(gpu):
+    """A half-rotated tensor whose packed form passes 4 GiB (1.2 GB in FP32) is still contracted on
+    chip: no buffer for T is allocated, and the result agrees with the GEMM path."""
+    afq, torch = gpu
+    N = n = 33
+    M, W = 281_000, 3
+    say(f"case: fused exchange, packed tensor past 4 GiB, N={N} n={n} M={M} W={W}")
+    g = torch.Generator(device="cuda").manual_seed(9)
+    L = torch.randn(N, N, M, generator=g, dtype=torch.float64, device="cuda") / N
+    L = (0.5 * (L + L.transpose(0, 1))).cpu().numpy()
+    rng = np.random.default_rng(9)
+    h1 = rng.normal(size=(N, N))
+    h1 = 0.5 * (h1 + h1.T)
+    PsiT = np.ascontiguousarray(np.linalg.qr(rng.normal(size=(N, N)))[0].astype(np.complex128))
+    ctx = afq.Context(0)
+    ham = afq.HamiltonianOperations(ctx, h1, L, PsiT, n, precision=afq.AFQ_MIXED)
+    del L
+    G = afq.device_tensor(rng.normal(size=(W, n, N)) + 1j * rng.normal(size=(W, n, N)))
+    before = ctx.scratch_bytes()
+    fused = _energies(afq, torch, ham, G, W, afq.AFQ_MIXED, fused=True)
+    grown = ctx.scratch_bytes() - before
+    say(f"  scratch grown by {grown >> 20} MiB")
+    assert grown < 256 << 20
+    gemm = _energies(afq, torch, ham, G, W, afq.AFQ_MIXED, fused=False)
+    for k in (1, 2):
+        assert per_walker(fused[:, k], gemm[:, k]) < BOUND
+
+
+def test_walker_runs(gpu):
+    """More walkers than one launch takes (their packed G passes 2 GiB): the last ones have the bits
+    that they have on their own."""
+    afq, torch = gpu
+    N, n, M, W = 33, 33, 5, 70_100
+    say(f"case: fused exchange, walker runs, N={N} n={n} M={M} W={W}")
+    p = make_problem(N, n, M, seed=78)
+    ctx = afq.Context(0)
+    ham = afq.HamiltonianOperations(ctx, p.h1, p.Likn, p.PsiT, n, precision=afq.AFQ_MIXED)
+    g = torch.Generator(device="cuda").manual_seed(11)
+    G = torch.randn(W, n, N, generator=g, dtype=torch.complex128, device="cuda")
+    every = _energies(afq, torch, ham, G, W, afq.AFQ_MIXED)
+    last = _energies(afq, torch, ham, G[-201:].contiguous(), 201, afq.AFQ_MIXED)
+    assert np.array_equal(every[-201:], last)
