@@ -43,6 +43,7 @@
 // 13.4 -> 11.3 us, N = 160, n = 40, 256 walkers 192 -> 179 us (its pieces spill).  So every size and
 // both kinds of P1 that fit take this kernel.
 #include <cstdlib>
+#include <type_traits>
 
 #include "ops.hpp"
 #include "split3.hpp"
@@ -374,17 +375,26 @@ __device__ inline void write_share(char* lds, int KG, int N, const Share<SLOTS>&
 template <int SLOTS, int WAVES>
 constexpr int kResident = SLOTS == 2 ? 1 : WAVES / 2;
 
+// A workgroup's part of the work
+struct Tile {
+  const float *P1, *V;  // V: this walker's
+  z64* Pw;
+  int N, n, c0, c1, order, e, wave;
+};
+
 // One wavefront's recurrence (FULL: it owns every block of its last stripe); every wavefront passes
-// the same barriers.
+// the same barriers.  False, with the walker as it was, where a sum is not finite.
 template <int P, int X, int SLOTS, int WAVES, bool P1C, bool FULL>
-__device__ inline void recur(Rows<P1C, true, kResident<SLOTS, WAVES>, SLOTS>& rp,
-                             Rows<true, false, kResident<SLOTS, WAVES>, SLOTS>& rv, int N, int n,
-                             int KG, int order, z64* Pw, int c0, int c1, const Share<SLOTS>& sh,
-                             int fr, int fk, char* lds, int e) {
+__device__ inline bool recur(Rows<P1C, true, kResident<SLOTS, WAVES>, SLOTS>& rp,
+                             Rows<true, false, kResident<SLOTS, WAVES>, SLOTS>& rv, int KG,
+                             const Tile& a, const Share<SLOTS>& sh, int& fr, int& fk,
+                             uint32_t* votes, char* lds) {
   // the running sum takes the rounded term, whichever way a block is laid out
 #pragma clang fp contract(off)
   constexpr int RES = kResident<SLOTS, WAVES>;
   constexpr bool SUM0 = SLOTS == 1;
+  const int N = a.N, n = a.n, order = a.order, c0 = a.c0, c1 = a.c1, e = a.e;
+  z64* Pw = a.Pw;
   Accs<P, X, SLOTS> acc, S;
   // T_0 = P1 Phi, S = T_0
   __syncthreads();
@@ -451,7 +461,22 @@ __device__ inline void recur(Rows<P1C, true, kResident<SLOTS, WAVES>, SLOTS>& rp
   }
   rp.start(KG);
   asm volatile("" : "+v"(fr), "+v"(fk));
+  // (x 0 is 0 for every finite x)
+  f32x4 z = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < SLOTS; ++s) {
+#pragma unroll
+    for (int t = 0; t < P; ++t)
+      if (sh.mask[s] >> t & 1u) z += S[s].re[t] * 0.f + S[s].im[t] * 0.f;
+    if (X && (sh.mask[s] >> P & 1u)) z += S[s].mx * 0.f;
+  }
+  const bool bad = __ballot(!((z[0] + z[1]) + (z[2] + z[3]) == 0.f)) != 0;
+  if (fr + fk == 0) votes[a.wave] = bad;
   __syncthreads();
+  bool any = false;
+#pragma unroll
+  for (int i = 0; i < WAVES; ++i) any = any || votes[i];
+  if (__ballot(any) != 0) return false;  // uniform per workgroup
   write_share<P, X, SLOTS>(lds, KG, N, sh, fr, fk, S);
   __syncthreads();
   // Phi = P1 S, scaled back by 2^e
@@ -465,6 +490,9 @@ __device__ inline void recur(Rows<P1C, true, kResident<SLOTS, WAVES>, SLOTS>& rp
       add_unit(acc[s].im[t], S[s].im[t], rp.unit[s], fk);
     }
     if constexpr (X) add_unit(acc[s].mx, S[s].mx, rp.unit[s], fk);
+  }
+#pragma unroll
+  for (int s = 0; s < SLOTS; ++s) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int row = sh.st[s] * 16 + 4 * fk + r;
@@ -483,16 +511,115 @@ __device__ inline void recur(Rows<P1C, true, kResident<SLOTS, WAVES>, SLOTS>& rp
       }
     }
   }
+  return true;
 }
 
-// P1C: complex P1
+// The workgroup's columns from plain FP32 products, for a walker whose sum came out infinite or NaN: the
+// split turns an infinity into NaN.  (A NaN in V or P1, or in a column, makes NaN of all its columns,
+// or of that one, in any arithmetic, without products.)  Columns by halves, so that the term, its
+// successor and the running sum fit where the pieces lay.  A function of its own, called when nothing
+// else is live: inlined, or with the sums kept across it, its registers cost the kernel 1 to 25 %.  One
+// infinite walker of 1024 (N = 200, n = 40) takes 3.0 ms instead of 0.87, 100 of them 4.1.
+template <int P, int X, int WAVES, bool P1C>
+__device__ __attribute__((noinline)) void redo_plain(Tile a, int tid, uint32_t* votes, char* lds) {
+#pragma clang fp contract(off)
+  constexpr int NC = 16 * P + 8 * X, H = NC / 2, TH = 64 * WAVES;
+  const int N = a.N;
+  auto vote = [&](bool v) {
+    const bool mine = __ballot(v) != 0;
+    __syncthreads();
+    if ((tid & 63) == 0) votes[tid >> 6] = mine;
+    __syncthreads();
+    bool any = false;
+    for (int i = 0; i < WAVES; ++i) any = any || votes[i];
+    return __ballot(any) != 0;
+  };
+  // a column without a NaN
+  bool clean = false;
+  for (int c = tid; c < a.c1 - a.c0; c += TH) {
+    bool nan = false;
+    for (int k = 0; k < N; ++k) {
+      const z64 v = a.Pw[(long)k * a.n + a.c0 + c];
+      nan = nan || v.re != v.re || v.im != v.im;
+    }
+    clean = clean || !nan;
+  }
+  bool products = vote(clean);
+  if (products) {
+    bool nan = false;
+    for (int t = tid; t < 2 * N * N; t += TH) {
+      nan = nan || a.V[t] != a.V[t];
+      if (P1C || t < N * N) nan = nan || a.P1[t] != a.P1[t];
+    }
+    products = !vote(nan);
+  }
+  if (!products) {
+    const double nan = __builtin_nan("");
+    for (int t = tid; t < N * (a.c1 - a.c0); t += TH)
+      a.Pw[(long)(t / (a.c1 - a.c0)) * a.n + a.c0 + t % (a.c1 - a.c0)] = z64{nan, nan};
+    return;
+  }
+  float2* T = reinterpret_cast<float2*>(lds);
+  float2 *U = T + N * H, *S = U + N * H;
+  const double sc = ldexp(1.0, -a.e), sb = ldexp(1.0, a.e);
+  // element (row, c) of A T
+  auto dot = [&](const float* A, auto cplx, const float2* B, int row, int c) {
+    float re = 0.f, im = 0.f;
+    for (int k = 0; k < N; ++k) {
+      const float2 b = B[k * H + c];
+      if constexpr (decltype(cplx)::value) {
+        const float ar = A[2 * ((long)row * N + k)], ai = A[2 * ((long)row * N + k) + 1];
+        re = fmaf(-ai, b.y, fmaf(ar, b.x, re));
+        im = fmaf(ai, b.x, fmaf(ar, b.y, im));
+      } else {
+        const float ar = A[(long)row * N + k];
+        re = fmaf(ar, b.x, re);
+        im = fmaf(ar, b.y, im);
+      }
+    }
+    return float2{re, im};
+  };
+  for (int h = 0; h < NC; h += H) {
+    __syncthreads();
+    for (int t = tid; t < N * H; t += TH) {
+      const int col = a.c0 + h + t % H;
+      const z64 v = col < a.c1 ? a.Pw[(long)(t / H) * a.n + col] : z64{0.0, 0.0};
+      T[t] = float2{(float)(v.re * sc), (float)(v.im * sc)};
+    }
+    __syncthreads();
+    for (int t = tid; t < N * H; t += TH)
+      S[t] = U[t] = dot(a.P1, std::bool_constant<P1C>{}, T, t / H, t % H);
+    for (int k = 1; k <= a.order; ++k) {
+      const float f = (float)(1.0 / (double)k);
+      __syncthreads();
+      for (int t = tid; t < N * H; t += TH) {
+        const float2 x = dot(a.V, std::true_type{}, U, t / H, t % H);
+        T[t] = float2{-(f * x.y), f * x.x};
+        S[t].x += T[t].x;
+        S[t].y += T[t].y;
+      }
+      float2* const o = T;
+      T = U;
+      U = o;
+    }
+    __syncthreads();
+    for (int t = tid; t < N * H; t += TH) {
+      const int col = a.c0 + h + t % H;
+      const float2 x = dot(a.P1, std::bool_constant<P1C>{}, S, t / H, t % H);
+      if (col < a.c1) a.Pw[(long)(t / H) * a.n + col] = z64{(double)x.x * sb, (double)x.y * sb};
+    }
+  }
+}
+
+// P1C: complex P1.  (The last bound keeps three workgroups a CU where 168 registers allow them.)
 template <int P, int X, int SLOTS, int WAVES, bool P1C>
-__global__ void __launch_bounds__(64 * WAVES, 2)
+__global__ void __launch_bounds__(64 * WAVES, WAVES == 4 && P == 1 && !P1C ? 3 : 2)
     k_prop_split(int W, int N, int n, int nchunk, int order, const float* __restrict__ P1,
                  const float* __restrict__ V, long v_bs, z64* __restrict__ Phi, long phi_bs) {
   constexpr int NC = 16 * P + 8 * X;
   extern __shared__ __align__(16) char lds[];
   __shared__ double wmx[WAVES];
+  __shared__ uint32_t votes[WAVES];
   const int NS = (N + 15) / 16, KG = (N + 31) / 32;
   const long total = gridDim.x, xcd = blockIdx.x % 8, slot = blockIdx.x / 8;
   const long q = xcd * (total / 8) + min(xcd, total % 8) + slot;
@@ -500,7 +627,7 @@ __global__ void __launch_bounds__(64 * WAVES, 2)
   // this workgroup's columns: the n columns in nchunk runs of whole 8-column groups
   const int n8 = (n + 7) / 8, c0 = 8 * (n8 * ch / nchunk), c1 = min(n, 8 * (n8 * (ch + 1) / nchunk));
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int fr = lane & 15, fk = lane >> 4;
+  int fr = lane & 15, fk = lane >> 4;
   z64* Pw = Phi + (long)w * phi_bs;
   const float* Vw = V + 2 * (long)w * v_bs;
 
@@ -585,10 +712,14 @@ __global__ void __launch_bounds__(64 * WAVES, 2)
     for (int x = 0; x < 3; ++x) *reinterpret_cast<bf16x8*>(o + x * s3::kPlane) = p[x];
   }
 
+  const Tile a{P1, Vw, Pw, N, n, c0, c1, order, e, wave};
+  bool done;
   if (sh.mask[SLOTS - 1] == ALL)
-    recur<P, X, SLOTS, WAVES, P1C, true>(rp, rv, N, n, KG, order, Pw, c0, c1, sh, fr, fk, lds, e);
+    done = recur<P, X, SLOTS, WAVES, P1C, true>(rp, rv, KG, a, sh, fr, fk, votes, lds);
   else
-    recur<P, X, SLOTS, WAVES, P1C, false>(rp, rv, N, n, KG, order, Pw, c0, c1, sh, fr, fk, lds, e);
+    done = recur<P, X, SLOTS, WAVES, P1C, false>(rp, rv, KG, a, sh, fr, fk, votes, lds);
+  if (__ballot(!done) != 0)  // uniform per workgroup
+    redo_plain<P, X, WAVES, P1C>(a, 64 * wave + 16 * fk + fr, votes, lds);
 }
 
 template <int P, int X, int SLOTS, int WAVES>

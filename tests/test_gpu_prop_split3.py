@@ -112,3 +112,77 @@ def test_walkers_past_fp32_range(gpu):
     got = propagate(afq, ctx, P1, V3, np.repeat(Phi, 3, axis=0) * s)
     assert np.array_equal(got[1] / 2.0 ** 130, got[0])
     assert np.array_equal(got[2] * 2.0 ** 130, got[0])
+
+
+def plain(P1, V, Phi, order):
+    """The recurrence in float64 with every complex product as four real ones, k by k, so that an
+    infinity times a zero part is the NaN that the FP32 products give."""
+    def mul(a, b, sign=1.0):
+        ar, ai, br, bi = a.real, a.imag, b.real, b.imag
+
+        def dot(x, y):
+            return (x[:, :, None] * y[None]).sum(axis=1)
+        with np.errstate(all="ignore"):
+            return dot(ar, br) - dot(ai, bi), dot(ar, bi) + dot(ai, br)
+
+    def z(re, im):
+        out = np.empty(re.shape, np.complex128)
+        out.real, out.imag = re, im
+        return out
+    T = z(*mul(P1, Phi))
+    S = T.copy()
+    for k in range(1, order + 1):
+        re, im = mul(V, T)
+        T = z(-(im / k), re / k)
+        with np.errstate(all="ignore"):
+            S = z(S.real + T.real, S.imag + T.imag)
+    return z(*mul(P1, S))
+
+
+@pytest.mark.parametrize("N,n", [(1, 1), (7, 3), (40, 21), (97, 23), (150, 12), (200, 40)])
+@pytest.mark.parametrize("order", [1, 2, 6])
+def test_infinities_and_nan(gpu, N, n, order):
+    """Infinities and NaN in the walkers, in V and in P1: infinite and NaN where the products in
+    FP32 are.  The other walkers keep their bits, the other columns of a walker with such a column
+    their values (1e-5 of the largest: FP32 products of at most 200 terms, four to eight of them)."""
+    afq, ctx, torch = gpu
+    print(f"case: split propagation with infinities N={N} n={n} order={order}", flush=True)
+    P1, V, Phi = inputs(N, n, 6)
+    Phi[:] /= np.abs(Phi).max(axis=(1, 2), keepdims=True)
+    clean = propagate(afq, ctx, P1, V, Phi, order)
+    inf, nan = np.inf, np.nan
+    A, B = V.copy(), Phi.copy()
+    B[0, N - 1, n - 1] = complex(inf, 0.5)
+    B[1, 0, 0] = complex(0.5, nan)
+    A[2, N // 2, 0] = complex(-inf, 0.5)
+    A[3, 0, N - 1] = complex(0.5, nan)
+    got = propagate(afq, ctx, P1, A, B, order)
+    assert np.array_equal(got[4:], clean[4:])
+    if n > 1:
+        for w, cols in ((0, np.s_[:n - 1]), (1, np.s_[1:])):
+            assert np.max(np.abs(got[w][:, cols] - clean[w][:, cols])) < 1e-5 * np.max(np.abs(clean[w]))
+    for w in range(4):
+        ref = plain(P1, A[w].astype(np.complex128), B[w], order)
+        for x, y in ((got[w].real, ref.real), (got[w].imag, ref.imag)):
+            assert np.array_equal(np.isnan(x), np.isnan(y)), w
+            m = np.isinf(y)
+            assert np.array_equal(np.isinf(x), m) and np.array_equal(x[m], y[m]), w
+    Q = P1.copy()
+    Q[N // 3, N // 2] = complex(inf, 1.0)
+    got = propagate(afq, ctx, Q, V, Phi, order)
+    for w in range(6):
+        ref = plain(Q, V[w].astype(np.complex128), Phi[w], order)
+        for x, y in ((got[w].real, ref.real), (got[w].imag, ref.imag)):
+            assert np.array_equal(np.isnan(x), np.isnan(y)), w
+            m = np.isinf(y)
+            assert np.array_equal(np.isinf(x), m) and np.array_equal(x[m], y[m]), w
+
+
+def test_overflow(gpu):
+    """A Taylor term past FP32's range: T_0 = 1.5, T_1 = (0, 4.5e38) becomes (0, inf) and leaves
+    P1 (1.5, inf) = (1.5 - 0 inf, inf + 0) = (NaN, inf)."""
+    afq, ctx, torch = gpu
+    print("case: split propagation past FP32's range", flush=True)
+    got = propagate(afq, ctx, np.ones((1, 1), np.complex128),
+                    np.full((1, 1, 1), 3e38, np.complex64), np.full((1, 1, 1), 1.5 + 0j), 1)[0, 0, 0]
+    assert np.isnan(got.real) and got.imag == np.inf
