@@ -180,9 +180,12 @@ inline bool fits(long rows, long K, bool cplx_rows) {
 // Pack a complex operand [rows][ld] (values rounded to FP32), or the rows of a real one; *bad is
 // set when a value of a real operand is not finite.  pack_pairs: row n is the orbital pair
 // pairs[n] = i << 16 | k of an [N * N][K] tensor.
-void pack_cplx(hipStream_t s, int rows, int K, const c32* X, long ld, void* out);
-void pack_cplx(hipStream_t s, int rows, int K, const z64* X, long ld, void* out);
-void pack_rows(hipStream_t s, int rows, int K, const float* X, long ld, void* out, int* bad);
+// Rows of two parts, K0 and then K1 values (vbias: the spins), start a new group with the second; a
+// real operand's parts are packed one by one, at group g0 of rows of ldg groups.
+void pack_cplx(hipStream_t s, int rows, int K0, int K1, const c32* X, long ld, void* out);
+void pack_cplx(hipStream_t s, int rows, int K0, int K1, const z64* X, long ld, void* out);
+void pack_rows(hipStream_t s, int rows, int K, const float* X, long ld, void* out, long ldg,
+               long g0, int* bad);
 void pack_pairs(hipStream_t s, int rows, int K, const float* X, int N, const uint32_t* pairs,
                 void* out, int* bad);
 // The operands of the exchange kernel (n <= 40): tiles of two walkers (G [W][n][N], real parts then
@@ -201,14 +204,15 @@ void pack_exx_L(hipStream_t s, int M, int n, int N, const float* L, void* out, i
 // to the first
 void vhs_pairs(hipStream_t s, int W, int np, int K, const void* A, const void* B,
                const uint32_t* pairs, int N, float alpha, c32* V);
-// v[w][m] (+)= alpha sum_k A[w][k] B[m][k], K cut into p.ksplit slices (ws [ksplit][W][M] when
-// more than one)
+// v[w][m] = alpha sum_k A[w][k] B[m][k] over both parts of the rows, by the plan's tile and K slices:
+// slices of kchunk groups, ks0 of the first part and the rest of the second; ws holds ksplit W M
+// values where there is more than one
 struct Plan {
-  int tile, ksplit, kchunk;
+  int tile, ksplit, kchunk, ks0;
 };
-Plan plan(int M, int N, int KG, bool split_k);
-void vbias(hipStream_t s, int W, int M, int K, const void* A, const void* B, const Plan& p,
-           float alpha, bool accumulate, z64* v, c32* ws);
+Plan vbias_plan(int W, int M, int K0, int K1);
+void vbias(hipStream_t s, int W, int M, int K0, int K1, const Plan& p, const void* A,
+           const void* B, float alpha, z64* v, c32* ws);
 }  // namespace s3
 
 }  // namespace afq

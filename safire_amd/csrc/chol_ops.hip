@@ -106,8 +106,6 @@ CholeskyOps::CholeskyOps(Context& c, int walker_type, int N, int nup, int ndown,
     Lnak_r32_ = own.Lnak_r32;
     Lnak32_ = own.Lnak32;
     Lnak_s3_ = own.Lnak_s3;
-    s3_off_[0] = own.s3_off[0];
-    s3_off_[1] = own.s3_off[1];
     Lexx_s3_[0] = own.Lexx_s3[0];
     Lexx_s3_[1] = own.Lexx_s3[1];
     real_trial_ = own.real;
@@ -205,14 +203,14 @@ void CholeskyOps::build_split(Rotated& r, bool own) const {
   const int N = N_, M = M_, ns[2] = {nup_, ndown_};
   int* bad = scratch_as<int>(ctx_, "setup_bad", 1);
   AFQ_HIP(hipMemsetAsync(bad, 0, sizeof(int), s));
-  r.s3_off[1] = s3::bytes_real(M, (long)nup_ * N);
+  const long kg0 = s3::k_groups((long)nup_ * N), ldg = kg0 + s3::k_groups((long)ndown_ * N);
   if (own && s3::fits(M, (long)std::max(nup_, ndown_) * N, false))
-    r.Lnak_s3 = dalloc<char>(r.s3_off[1] + s3::bytes_real(M, (long)ndown_ * N));
+    r.Lnak_s3 = dalloc<char>((size_t)(s3::row_blocks(M) * ldg * s3::kBlock));
   for (int sp = 0; sp < 2; ++sp) {
     if (ns[sp] == 0) continue;
     const float* L = r.Lnak_r32 + (sp == 0 ? 0 : (size_t)M * nup_ * N);
     if (r.Lnak_s3)
-      s3::pack_rows(s, M, ns[sp] * N, L, (long)ns[sp] * N, r.Lnak_s3 + r.s3_off[sp], bad);
+      s3::pack_rows(s, M, ns[sp] * N, L, (long)ns[sp] * N, r.Lnak_s3, ldg, sp == 0 ? 0 : kg0, bad);
     if (std::max(nup_, ndown_) <= 40 && (size_t)M * ns[sp] * N * sizeof(float) < (1UL << 32)) {
       r.Lexx_s3[sp] = dalloc<char>(s3::bytes_exx_L(M, ns[sp], N));
       s3::pack_exx_L(s, M, ns[sp], N, L, r.Lexx_s3[sp], bad);
@@ -390,7 +388,7 @@ void CholeskyOps::vHS(const void* X, int W, double dt, void* V, Precision prec) 
           // on the bfloat16 matrix cores over the N(N+1)/2 distinct pairs, k groups from the
           // last Cholesky vector to the first
           const int np = N_ * (N_ + 1) / 2;
-          if (l == 0) s3::pack_cplx(s, W, M_, X32, M_, A);
+          if (l == 0) s3::pack_cplx(s, W, M_, 0, X32, M_, A);
           s3::vhs_pairs(s, W, np, M_, A, Lpair_s3_ + l * s3::bytes_real(np, M_), pairs_, N_,
                         (float)a, reinterpret_cast<c32*>(Vl));
         } else {
@@ -428,6 +426,26 @@ void CholeskyOps::vbias_f32(const cplx<TG>* G, int W, double dt, z64* v) const {
   hipStream_t s = ctx_.stream();
   const float a = (float)(std::sqrt(dt) * (walker_type_ == kClosed ? 2.0 : 1.0));
   const int nel_ = nel();
+  const int K0 = nup_ * N_, K1 = ndown_ * N_;  // the spins' values of a row of G
+  if (Lnak_s3_ && nel_ > 0 && crg_path()) {
+    // on the bfloat16 matrix cores, both spins in one product, K cut into slices so that the tiles
+    // fill the machine; the walkers in runs that the 32-bit offsets reach
+    const size_t per16 = s3::bytes_cplx(16, K0) + s3::bytes_cplx(16, K1);
+    const int run = (int)std::min<size_t>((size_t)W, 16 * std::max<size_t>(1, 0xFFFF0000u / per16));
+    void* Gp = ctx_.scratch_kept("s3_G", (size_t)s3::row_blocks(run) * per16);
+    const s3::Plan p = s3::vbias_plan(run, M_, K0, K1);
+    void* ws = ctx_.scratch_kept("s3_ws", p.ksplit > 1 ? sizeof(c32) * p.ksplit * run * M_ : 1);
+    if (Gp && ws) {
+      for (int w = 0; w < W; w += run) {
+        const int wc = std::min(run, W - w);
+        const cplx<TG>* Gw = G + (size_t)w * nel_ * N_;
+        s3::pack_cplx(s, wc, K0, K1, Gw, (long)nel_ * N_, Gp);
+        s3::vbias(s, wc, M_, K0, K1, p, Gp, Lnak_s3_, a, v + (size_t)w * M_,
+                  static_cast<c32*>(ws));
+      }
+      return;
+    }
+  }
   for (int sp = 0; sp < (walker_type_ == kCollinear ? 2 : 1); ++sp) {
     int ns = sp == 0 ? nup_ : ndown_;
     int acc = (sp == 1 && nup_ > 0) ? 1 : 0;
@@ -439,17 +457,6 @@ void CholeskyOps::vbias_f32(const cplx<TG>* G, int W, double dt, z64* v) const {
     size_t loff = sp == 0 ? 0 : (size_t)M_ * nup_ * N_;
     const long K = (long)ns * N_;
     EpiStore<float, double> e{v, M_, 0, a, 0.f, acc};
-    char* Gp = nullptr;
-    if (Lnak_s3_ && crg_path() && s3::fits(W, K, true))
-      Gp = static_cast<char*>(ctx_.scratch_kept("s3_G", s3::bytes_cplx(W, K)));
-    if (Gp) {
-      // on the bfloat16 matrix cores, K cut into slices so that the tiles fill the machine
-      s3::pack_cplx(s, W, (int)K, G + goff, (long)nel_ * N_, Gp);
-      const s3::Plan p = s3::plan(W, M_, (int)s3::k_groups(K), true);
-      c32* ws = p.ksplit > 1 ? scratch_as<c32>(ctx_, "s3_ws", (size_t)p.ksplit * W * M_) : nullptr;
-      s3::vbias(s, W, M_, (int)K, Gp, Lnak_s3_ + s3_off_[sp], p, a, acc != 0, v, ws);
-      continue;
-    }
     constexpr bool g32 = sizeof(TG) == 4;
     Opnd<TG, true, true> A{&(G + goff)->re, (long)nel_ * N_, 0};
     if (real_trial_) {

@@ -141,9 +141,8 @@ struct Rotated {
   c32* Lnak32 = nullptr;      // FP32 copy (mixed precision, complex determinant)
   bool real = false;
   // mixed precision, the hamiltonian's own real determinant: Lnak_r32 split into bfloat16 pieces and
-  // packed for vbias (split3.hpp, one block per spin at s3_off); null when it does not apply
+  // packed for vbias (split3.hpp, a row per vector over both spins); null when it does not apply
   char* Lnak_s3 = nullptr;
-  size_t s3_off[2] = {0, 0};
   // and packed for the fused exchange (exchange.hip; electrons <= 40), one block per spin
   char* Lexx_s3[2] = {nullptr, nullptr};
 };
@@ -209,7 +208,7 @@ class CholeskyOps {
   // the hamiltonian's own determinant
   Rotated self() const {
     return Rotated{PsiT_, Lnak_, haj_, Lnak_r_, Lnak_r32_, Lnak32_, real_trial_, Lnak_s3_,
-                   {s3_off_[0], s3_off_[1]}, {Lexx_s3_[0], Lexx_s3_[1]}};
+                   {Lexx_s3_[0], Lexx_s3_[1]}};
   }
   // vMF (NOMSD.cpp:437-464) with the charge-decomposition zero_imag (AFQMCBasePropagator.cpp:105)
   void vMF(double dt, z64* v) const;
@@ -244,7 +243,6 @@ class CholeskyOps {
   char* Lpair_s3_ = nullptr;
   uint32_t* pairs_ = nullptr;
   char* Lnak_s3_ = nullptr;
-  size_t s3_off_[2] = {0, 0};
   char* Lexx_s3_[2] = {nullptr, nullptr};
   void build_pairs();
   // packs the FP32 half-rotated tensor for the exchange and (own) vbias (split3.hpp)

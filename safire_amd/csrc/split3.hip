@@ -17,26 +17,29 @@ namespace s3 {
 constexpr int kTiles = 4;
 constexpr int kTileRB[kTiles] = {2, 2, 2, 1}, kTileCB[kTiles] = {6, 5, 4, 6};
 
-Plan plan(int M, int N, int KG, bool split_k) {
+static Plan plan(int M, int N, int KG0, int KG1, bool split_k) {
   constexpr double kWeight[kTiles] = {1.0, 1.05, 1.15, 1.34};
-  Plan best{0, 1, KG};
+  const int KG = std::max(KG0, KG1);
+  Plan best{0, 1, KG, 1};
   double tb = 1e300;
   for (int t = 0; t < kTiles; ++t) {
     const int rb = kTileRB[t], cb = kTileCB[t];
     const long tiles = (long)ceil_div(M, 16 * rb) * ceil_div(N, 16 * cb);
     const int cap = split_k ? std::max(1, std::min(KG / 4, 16)) : 1;
-    for (int ks = 1; ks <= cap; ++ks) {
-      const int kc = ceil_div(KG, ks);
-      if (ceil_div(KG, kc) != ks) continue;
+    for (int c = 1; c <= cap; ++c) {
+      const int kc = ceil_div(KG, c);
+      if (ceil_div(KG, kc) != c) continue;
+      const int ks0 = ceil_div(KG0, kc), ks = ks0 + ceil_div(KG1, kc);
+      if (c > 1 && ks > 16) continue;
       const long per_simd = (tiles * ks + 1023) / 1024;
       // 12 MFMAs of 16 cycles per block and k group; partials: 16 bytes per element and slice at
       // about 2 bytes a cycle and SIMD
-      double c = (double)per_simd * rb * cb * kc * 12 * 16 * kWeight[t];
-      if (per_simd == 1) c *= 1.15;
-      if (ks > 1) c += 4000.0 + 16.0 * ks * M * (double)N / 2048.0;
-      if (c < tb * 0.999) {
-        tb = c;
-        best = Plan{t, ks, kc};
+      double x = (double)per_simd * rb * cb * kc * 12 * 16 * kWeight[t];
+      if (per_simd == 1) x *= 1.15;
+      if (ks > 1) x += 4000.0 + 16.0 * ks * M * (double)N / 2048.0;
+      if (x < tb * 0.999) {
+        tb = x;
+        best = Plan{t, ks, kc, ks0};
       }
     }
   }
@@ -46,60 +49,62 @@ Plan plan(int M, int N, int KG, bool split_k) {
 namespace {
 
 template <typename TIn, class ROWS>
-void pack_cplx_t(hipStream_t s, long blocks, int K, const cplx<TIn>* X, long ld, const ROWS& rmap,
-                 int nb, void* out) {
-  const long KG = k_groups(K), waves = blocks * KG;
+void pack_cplx_t(hipStream_t s, long blocks, int K0, int K1, const cplx<TIn>* X, long ld,
+                 const ROWS& rmap, int nb, void* out) {
+  const long KG = k_groups(K0) + k_groups(K1), waves = blocks * KG;
   if (waves == 0) return;
   AFQ_CHECK((waves + 3) / 4 < (1L << 31), kErrShape, "grid too large");
   hipLaunchKernelGGL((k_pack_cplx<TIn, ROWS>), dim3((unsigned)ceil_div(waves, 4)), dim3(256), 0, s,
-                     blocks, K, (int)KG, X, ld, rmap, nb, static_cast<char*>(out));
+                     blocks, K0, (int)k_groups(K0), K0 + K1, (int)KG, X, ld, rmap, nb,
+                     static_cast<char*>(out));
   AFQ_LAUNCH_CHECK();
 }
 
 template <class ROWS>
 void pack_real_t(hipStream_t s, long blocks, int K, const float* X, long ld, const ROWS& rmap,
-                 void* out, int* bad) {
+                 void* out, long ldg, long g0, int* bad) {
   const long KG = k_groups(K), waves = blocks * KG;
   if (waves == 0) return;
   AFQ_CHECK((waves + 3) / 4 < (1L << 31), kErrShape, "grid too large");
   hipLaunchKernelGGL((k_pack_real<ROWS>), dim3((unsigned)ceil_div(waves, 4)), dim3(256), 0, s,
-                     blocks, K, (int)KG, X, ld, rmap, static_cast<char*>(out), bad);
+                     blocks, K, (int)KG, X, ld, rmap, static_cast<char*>(out), (int)ldg, (int)g0,
+                     bad);
   AFQ_LAUNCH_CHECK();
 }
 
 template <int RB, int CB, bool REVK, class EPI>
-void launch_tile(hipStream_t s, int M, int N, int KG, const void* A, const void* B, int ksplit,
-                 int kchunk, const EPI& e) {
+void launch_tile(hipStream_t s, int M, int N, int KG, int KG0, const void* A, const void* B,
+                 const Plan& p, const EPI& e) {
   const int tm = ceil_div(M, 16 * RB), tn = ceil_div(N, 16 * CB);
-  const long blocks = ceil_div((long)tm * tn * ksplit, 4);
+  const long blocks = ceil_div((long)tm * tn * p.ksplit, 4);
   AFQ_CHECK(blocks < (1L << 31), kErrShape, "grid too large");
   hipLaunchKernelGGL((k_split3_gemm<RB, CB, REVK, EPI>), dim3((unsigned)blocks), dim3(256), 0, s, M,
-                     N, KG, static_cast<const char*>(A), static_cast<const char*>(B), tm, tn, ksplit,
-                     kchunk, e);
+                     N, KG, KG0, static_cast<const char*>(A), static_cast<const char*>(B), tm, tn,
+                     p.ksplit, p.ks0, p.kchunk, e);
   AFQ_LAUNCH_CHECK();
 }
 
 template <bool REVK, class EPI>
-void launch_planned(hipStream_t s, int M, int N, int KG, const void* A, const void* B,
+void launch_planned(hipStream_t s, int M, int N, int KG, int KG0, const void* A, const void* B,
                     const Plan& p, const EPI& e) {
   switch (p.tile) {
-    case 0: launch_tile<2, 6, REVK>(s, M, N, KG, A, B, p.ksplit, p.kchunk, e); break;
-    case 1: launch_tile<2, 5, REVK>(s, M, N, KG, A, B, p.ksplit, p.kchunk, e); break;
-    case 2: launch_tile<2, 4, REVK>(s, M, N, KG, A, B, p.ksplit, p.kchunk, e); break;
-    default: launch_tile<1, 6, REVK>(s, M, N, KG, A, B, p.ksplit, p.kchunk, e); break;
+    case 0: launch_tile<2, 6, REVK>(s, M, N, KG, KG0, A, B, p, e); break;
+    case 1: launch_tile<2, 5, REVK>(s, M, N, KG, KG0, A, B, p, e); break;
+    case 2: launch_tile<2, 4, REVK>(s, M, N, KG, KG0, A, B, p, e); break;
+    default: launch_tile<1, 6, REVK>(s, M, N, KG, KG0, A, B, p, e); break;
   }
 }
 
 // C = epi(A B^T): one launch, or K slices whose FP32 partials (ws [ksplit][M][N]) are summed in
 // slice order in FP64 before the epilogue.
 template <bool REVK, class EPI>
-void product_splitk(hipStream_t s, int M, int N, int KG, const void* A, const void* B,
+void product_splitk(hipStream_t s, int M, int N, int KG, int KG0, const void* A, const void* B,
                     const Plan& p, const EPI& e, c32* ws) {
   if (p.ksplit == 1) {
-    launch_planned<REVK>(s, M, N, KG, A, B, p, Plain<EPI>{e});
+    launch_planned<REVK>(s, M, N, KG, KG0, A, B, p, Plain<EPI>{e});
     return;
   }
-  launch_planned<REVK>(s, M, N, KG, A, B, p,
+  launch_planned<REVK>(s, M, N, KG, KG0, A, B, p,
                        Plain<gemm::EpiPartial<float>>{{ws, (long)M * N, N}});
   const long tot = (long)M * N;
   hipLaunchKernelGGL((gemm::kreduce_splitk<float, EPI>), dim3((unsigned)ceil_div(tot, 256)),
@@ -109,38 +114,52 @@ void product_splitk(hipStream_t s, int M, int N, int KG, const void* A, const vo
 
 }  // namespace
 
-void pack_cplx(hipStream_t s, int rows, int K, const c32* X, long ld, void* out) {
-  pack_cplx_t(s, row_blocks(rows), K, X, ld, RowsPlain{rows}, 1, out);
+void pack_cplx(hipStream_t s, int rows, int K0, int K1, const c32* X, long ld, void* out) {
+  pack_cplx_t(s, row_blocks(rows), K0, K1, X, ld, RowsPlain{rows}, 1, out);
 }
-void pack_cplx(hipStream_t s, int rows, int K, const z64* X, long ld, void* out) {
-  pack_cplx_t(s, row_blocks(rows), K, X, ld, RowsPlain{rows}, 1, out);
+void pack_cplx(hipStream_t s, int rows, int K0, int K1, const z64* X, long ld, void* out) {
+  pack_cplx_t(s, row_blocks(rows), K0, K1, X, ld, RowsPlain{rows}, 1, out);
 }
-void pack_rows(hipStream_t s, int rows, int K, const float* X, long ld, void* out, int* bad) {
-  pack_real_t(s, row_blocks(rows), K, X, ld, RowsPlain{rows}, out, bad);
+void pack_rows(hipStream_t s, int rows, int K, const float* X, long ld, void* out, long ldg,
+               long g0, int* bad) {
+  pack_real_t(s, row_blocks(rows), K, X, ld, RowsPlain{rows}, out, ldg, g0, bad);
 }
 void pack_pairs(hipStream_t s, int rows, int K, const float* X, int N, const uint32_t* pairs,
                 void* out, int* bad) {
-  pack_real_t(s, row_blocks(rows), K, X, K, RowsPairs{pairs, rows, N}, out, bad);
+  pack_real_t(s, row_blocks(rows), K, X, K, RowsPairs{pairs, rows, N}, out, k_groups(K), 0, bad);
 }
 void pack_exx_G(hipStream_t s, int W, int n, int N, const z64* G, void* out) {
   const int nb = exx_nb(n);
-  pack_cplx_t(s, (long)ceil_div(W, 2) * nb, N, G, N, RowsItems{W, n, 8 * nb}, nb, out);
+  pack_cplx_t(s, (long)ceil_div(W, 2) * nb, N, 0, G, N, RowsItems{W, n, 8 * nb}, nb, out);
 }
 void pack_exx_L(hipStream_t s, int M, int n, int N, const float* L, void* out, int* bad) {
   const int nb = exx_nb(n);
-  pack_real_t(s, (long)ceil_div(M, 2) * nb, N, L, N, RowsItems{M, n, 8 * nb}, out, bad);
+  pack_real_t(s, (long)ceil_div(M, 2) * nb, N, L, N, RowsItems{M, n, 8 * nb}, out, k_groups(N), 0,
+              bad);
 }
 
 void vhs_pairs(hipStream_t s, int W, int np, int K, const void* A, const void* B,
                const uint32_t* pairs, int N, float alpha, c32* V) {
   const int KG = (int)k_groups(K);
-  launch_planned<true>(s, W, np, KG, A, B, plan(W, np, KG, false), EpiPairs{V, pairs, N, alpha, 0.f});
+  launch_planned<true>(s, W, np, KG, KG, A, B, plan(W, np, KG, 0, false),
+                       EpiPairs{V, pairs, N, alpha, 0.f});
 }
 
-void vbias(hipStream_t s, int W, int M, int K, const void* A, const void* B, const Plan& p,
-           float alpha, bool accumulate, z64* v, c32* ws) {
-  const gemm::EpiStore<float, double> e{v, M, 0, alpha, 0.f, accumulate ? 1 : 0};
-  product_splitk<false>(s, W, M, (int)k_groups(K), A, B, p, e, ws);
+Plan vbias_plan(int W, int M, int K0, int K1) {
+  return plan(W, M, (int)k_groups(K0), (int)k_groups(K1), true);
+}
+
+void vbias(hipStream_t s, int W, int M, int K0, int K1, const Plan& p, const void* A,
+           const void* B, float alpha, z64* v, c32* ws) {
+  const int KG0 = (int)k_groups(K0), KG = KG0 + (int)k_groups(K1);
+  // the vectors in runs that the 32-bit offsets reach
+  const long per = KG * kBlock;  // of 16 vectors
+  const int run = 16 * (int)std::max<long>(1, 0xFFFF0000L / per);
+  for (int m0 = 0; m0 < M; m0 += run) {
+    const gemm::EpiStore<float, double> e{v + m0, M, 0, alpha, 0.f, 0};
+    product_splitk<false>(s, W, std::min(run, M - m0), KG, KG0, A,
+                          static_cast<const char*>(B) + m0 / 16 * per, p, e, ws);
+  }
 }
 
 }  // namespace s3

@@ -117,20 +117,22 @@ struct RowsItems {
 // bound by memory.
 template <typename TIn, class ROWS>
 __global__ void __launch_bounds__(256)
-    k_pack_cplx(long blocks, int K, int KG, const cplx<TIn>* __restrict__ X, long ld, ROWS rmap,
-                int nb, char* __restrict__ out) {
+    k_pack_cplx(long blocks, int K0, int KG0, int K, int KG, const cplx<TIn>* __restrict__ X,
+                long ld, ROWS rmap, int nb, char* __restrict__ out) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const long q = (long)blockIdx.x * 4 + wave;
   const long rb = q / KG;
   const int kg = (int)(q % KG);
   if (rb >= blocks) return;
   const long r = rmap.src(16 * rb + (lane & 15));
-  const int k0 = 32 * kg + 8 * (lane >> 4);
+  // values [0, K0) fill the first KG0 groups, [K0, K) the others
+  const int k0 = 32 * kg + 8 * (lane >> 4) + (kg < KG0 ? 0 : K0 - 32 * KG0);
+  const int kn = kg < KG0 ? K0 : K;
   const cplx<TIn>* x = X + max(r, 0L) * ld + k0;
   float re[8], im[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
-    const cplx<TIn> v = (r >= 0 && k0 + j < K) ? x[j] : cplx<TIn>{0, 0};
+    const cplx<TIn> v = (r >= 0 && k0 + j < kn) ? x[j] : cplx<TIn>{0, 0};
     re[j] = (float)v.re;
     im[j] = (float)v.im;
   }
@@ -145,12 +147,12 @@ __global__ void __launch_bounds__(256)
   for (int c = 0; c < 3; ++c) *reinterpret_cast<u32x4*>(o + c * kPlane) = p[c];
 }
 
-// A real operand (built once per hamiltonian): one wavefront per (16-row block, k group).  *bad
-// is set when a value is not finite.
+// A real operand (built once per hamiltonian): one wavefront per (16-row block, k group), to the
+// groups from g0 on of rows of ldg groups.  *bad is set when a value is not finite.
 template <class ROWS>
 __global__ void __launch_bounds__(256)
     k_pack_real(long blocks, int K, int KG, const float* __restrict__ X, long ld, ROWS rmap,
-                char* __restrict__ out, int* __restrict__ bad) {
+                char* __restrict__ out, int ldg, int g0, int* __restrict__ bad) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const long q = (long)blockIdx.x * 4 + wave;
   const long rb = q / KG;
@@ -169,7 +171,7 @@ __global__ void __launch_bounds__(256)
   if (!fin) *bad = 1;
   u32x4 p[3];
   split8(v, p);
-  char* o = out + (rb * KG + kg) * kBlock + lane * 16;
+  char* o = out + (rb * ldg + g0 + kg) * kBlock + lane * 16;
 #pragma unroll
   for (int c = 0; c < 3; ++c) *reinterpret_cast<u32x4*>(o + c * kPlane) = p[c];
 }
@@ -314,7 +316,8 @@ __device__ inline void redo_non_finite(f32x4 (&c)[RA][CB], __amdgpu_buffer_rsrc_
 // Tiles run in strips two columns wide, so the four wavefronts of a workgroup form a 2 x 2 patch
 // and share both operands through L1; workgroups are renumbered so that each of the 8 XCDs takes
 // a contiguous run.  REVK: k groups from the last to the first (terms that fall with k are added
-// smallest first).  Split-K slices pass ks to the epilogue.
+// smallest first).  Split-K slices pass ks to the epilogue: ks0 slices of kchunk groups of the first
+// KG0 groups, then those of the others (the two spins of vbias, whose sums stay apart).
 //
 // Bound by the matrix cores and their operand feed through L2.  Measured (1024 x 20100 outputs
 // over 1600): 0.60 ms = 220 TFLOP/s of FP32 products, 0.57 of what six back-to-back MFMAs reach on
@@ -322,8 +325,9 @@ __device__ inline void redo_non_finite(f32x4 (&c)[RA][CB], __amdgpu_buffer_rsrc_
 // barrier per k group (more reuse in L1) measured 2-18 % slower.
 template <int RB, int CB, bool REVK, class EPI>
 __global__ void __launch_bounds__(256, 2)
-    k_split3_gemm(int M, int N, int KG, const char* __restrict__ A, const char* __restrict__ B,
-                  int tm, int tn, int ksplit, int kchunk, EPI epi) {
+    k_split3_gemm(int M, int N, int KG, int KG0, const char* __restrict__ A,
+                  const char* __restrict__ B, int tm, int tn, int ksplit, int ks0, int kchunk,
+                  EPI epi) {
   constexpr int RA = 2 * RB;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int fr = lane & 15, fk = lane >> 4;
@@ -336,7 +340,8 @@ __global__ void __launch_bounds__(256, 2)
   const int strip = t / (2 * tm), in0 = 2 * strip, wd = min(2, tn - in0), rem = t - strip * 2 * tm;
   const int im = rem / wd, in = in0 + rem % wd;
   const int m0 = 16 * RB * im, n0 = 16 * CB * in;
-  const int g0 = ks * kchunk, gn = min(KG - g0, kchunk);
+  const int g0 = ks < ks0 ? ks * kchunk : KG0 + (ks - ks0) * kchunk;
+  const int gn = min((ks < ks0 ? KG0 : KG) - g0, kchunk);
   const int rba = (M + 15) / 16, rbb = (N + 15) / 16;
   // blocks past the last row block read the last one; their results are never stored
   uint32_t oa[RA], ob[CB];

@@ -235,3 +235,28 @@ def test_captured_without_a_first_call(gpu, which):
                 assert np.array_equal(a, b)
             else:  # other kernels: 30 or 120 FP32 products of N(0, 1) numbers
                 assert np.max(np.abs(a - b)) < 1e-5 * np.max(np.abs(b))
+
+
+@pytest.mark.parametrize("N,n,nd,M,W", [(37, 9, 7, 150, 96), (64, 16, 16, 320, 256)])
+def test_two_spins_take_the_launches_of_one(gpu, N, n, nd, M, W):
+    """A two-spin vbias packs both density matrices in one launch and forms one product whose K slices
+    keep the spins apart: three launches at most (pack, product, sum of the slices)."""
+    import ctypes
+    afq, ctx, torch = gpu
+    print(f"case: launches of a two-spin vbias N={N} n={n}+{nd} M={M} W={W}", flush=True)
+    p = make_problem(N, n, M, 4)
+    ham = afq.HamiltonianOperations(ctx, p.h1, p.Likn, np.concatenate([p.PsiT, p.PsiT[:nd]]), n, nd,
+                                    walker_type=afq.AFQ_COLLINEAR, precision=afq.AFQ_MIXED)
+    G = torch.randn(W, n + nd, N, dtype=torch.complex128, device="cuda")
+    v = afq.empty((W, M), torch.complex128)
+    ham.vbias(G, v, 1.0)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(g, stream=ctx.stream):
+        ham.vbias(G, v, 1.0)
+    hip = ctypes.CDLL("libamdhip64.so")
+    nodes = ctypes.c_size_t(0)
+    assert hip.hipGraphGetNodes(ctypes.c_void_p(g.raw_cuda_graph()), None,
+                                ctypes.byref(nodes)) == 0
+    print("  nodes", nodes.value, flush=True)
+    assert 2 <= nodes.value <= 3
