@@ -595,12 +595,42 @@ __global__ void __launch_bounds__(256, RMAX <= 4 ? 2 : 1)
   }
 }
 
+// B determinants d0, d0 + 256, ... of a thread: the chain of index, weight and dot product of a single one
+// is bound by the latency of its loads
+template <int B>
+__device__ inline void ph_cross_dets(int d0, int ndet, int cn, const int* __restrict__ crow,
+                                     const int* __restrict__ ccol, const z64* __restrict__ cval,
+                                     const z64* oa, const z64* ob, const z64* sa, const z64* sb,
+                                     int ld, z64& acc) {
+  int u[B], v[B];
+  z64 wt[B], dot[B];
+#pragma unroll
+  for (int i = 0; i < B; ++i) {
+    const int d = min(d0 + 256 * i, ndet - 1);
+    u[i] = crow[d];
+    v[i] = ccol[d];
+    wt[i] = cval[d];
+    dot[i] = z64{0.0, 0.0};
+  }
+#pragma unroll
+  for (int i = 0; i < B; ++i) wt[i] = zmul(wt[i], zmul(oa[u[i]], ob[v[i]]));
+  for (int j = 0; j < cn; ++j)
+#pragma unroll
+    for (int i = 0; i < B; ++i) dot[i] = zfma(sa[u[i] * ld + j], sb[v[i] * ld + j], dot[i]);
+#pragma unroll
+  for (int i = 0; i < B; ++i)
+    if (d0 + 256 * i < ndet) acc = zfma(wt[i], dot[i], acc);
+}
+
 // Opposite-spin Coulomb coupling over Cholesky slices [n0, n0 + CH) of walker w:
 //   out[w][chunk] = sum_d conj(ci_d) ova[a_d] ovb[b_d] sum_n Ka[a_d][n] Kb[b_d][n]
-// with both spins' slices staged in LDS; determinants in alpha-row order (crow, cca, cva);
-// per-thread sums over a fixed set of determinants, then a fixed tree.
+// determinants in alpha-row order (crow, cca, cva); per-thread sums over a fixed set of determinants, then
+// a fixed tree.  LDS: both spins' slices staged, [na][ld] then [nb][ld]; else read in place, half a
+// row of each spin in flight.  Staging is bound by the reading of KE, reading in place by the latency of
+// the gathers (ph_cross_shape chooses).
+template <bool LDS>
 __global__ void __launch_bounds__(256)
-    k_ph_cross(int na, int nb, int M, int CH, int lds, int ndet, const int* __restrict__ crow,
+    k_ph_cross(int na, int nb, int M, int CH, int ld, int ndet, const int* __restrict__ crow,
                const int* __restrict__ ccol, const z64* __restrict__ cval,
                const z64* __restrict__ ova, const z64* __restrict__ ovb,
                const z64* __restrict__ KEa, const z64* __restrict__ KEb, z64* __restrict__ out) {
@@ -608,53 +638,67 @@ __global__ void __launch_bounds__(256)
   __shared__ z64 red[256];
   const int chunk = blockIdx.x, w = blockIdx.y, nch = gridDim.x, tid = threadIdx.x;
   const int n0 = chunk * CH, cn = min(CH, M - n0);
-  const z64* Ka = KEa + (long)w * na * M;
-  const z64* Kb = KEb + (long)w * nb * M;
-  // slices in LDS ([na][CH + 1] then [nb][CH + 1]) when they fit, else read in place
-  const z64* sa = Ka + n0;
-  const z64* sb = Kb + n0;
-  long ld = M;
-  if (lds) {
-    z64* da = sk;
-    z64* db = sk + (long)na * (CH + 1);
-    auto to = [&](int t) { return t + t / CH; };
-    stage_lds(da, na * CH,
-              [&](int t) { return Ka + (long)(t / CH) * M + n0 + min(t % CH, cn - 1); }, to);
-    stage_lds(db, nb * CH,
-              [&](int t) { return Kb + (long)(t / CH) * M + n0 + min(t % CH, cn - 1); }, to);
-    __syncthreads();
-    sa = da;
-    sb = db;
-    ld = CH + 1;
-  }
+  const z64* Ka = KEa + (long)w * na * M + n0;
+  const z64* Kb = KEb + (long)w * nb * M + n0;
   const z64* oa = ova + (long)w * na;
   const z64* ob = ovb + (long)w * nb;
   z64 acc = {0.0, 0.0};
-  // eight determinants at a time: the chain of index, weight and dot product of a single one is
-  // bound by the latency of its loads
-  constexpr int B = 8;
-  for (int d0 = tid; d0 < ndet; d0 += 256 * B) {
-    int u[B], v[B];
-    z64 wt[B], dot[B];
+  if constexpr (!LDS) {
+    for (int d = tid; d < ndet; d += 256) {
+      const int u = crow[d], v = ccol[d];
+      const z64* a = Ka + (long)u * M;
+      const z64* b = Kb + (long)v * M;
+      z64 dot = {0.0, 0.0};
+      int j = 0;
+      for (; j + 8 <= cn; j += 8) {
+        z64 x[8], y[8];
 #pragma unroll
-    for (int i = 0; i < B; ++i) {
-      const int d = min(d0 + 256 * i, ndet - 1);
-      u[i] = crow[d];
-      v[i] = ccol[d];
-      wt[i] = cval[d];
-      dot[i] = z64{0.0, 0.0};
+        for (int i = 0; i < 8; ++i) {
+          x[i] = a[j + i];
+          y[i] = b[j + i];
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) dot = zfma(x[i], y[i], dot);
+      }
+      for (; j < cn; ++j) dot = zfma(a[j], b[j], dot);
+      acc = zfma(zmul(cval[d], zmul(oa[u], ob[v])), dot, acc);
     }
-#pragma unroll
-    for (int i = 0; i < B; ++i) wt[i] = zmul(wt[i], zmul(oa[u[i]], ob[v[i]]));
-    for (int j = 0; j < cn; ++j)
-#pragma unroll
-      for (int i = 0; i < B; ++i) dot[i] = zfma(sa[u[i] * ld + j], sb[v[i] * ld + j], dot[i]);
-#pragma unroll
-    for (int i = 0; i < B; ++i)
-      if (d0 + 256 * i < ndet) acc = zfma(wt[i], dot[i], acc);
+  } else {
+    z64* da = sk;
+    z64* db = sk + (long)na * ld;
+    auto to = [&](int t) { return t / CH * ld + t % CH; };
+    stage_lds(da, na * CH, [&](int t) { return Ka + (long)(t / CH) * M + min(t % CH, cn - 1); },
+              to);
+    stage_lds(db, nb * CH, [&](int t) { return Kb + (long)(t / CH) * M + min(t % CH, cn - 1); },
+              to);
+    __syncthreads();
+    int d = tid;  // (d - tid: the workgroup's first)
+    for (; d - tid + 4 * 256 < ndet; d += 8 * 256)
+      ph_cross_dets<8>(d, ndet, cn, crow, ccol, cval, oa, ob, da, db, ld, acc);
+    for (; d - tid + 256 < ndet; d += 4 * 256)
+      ph_cross_dets<4>(d, ndet, cn, crow, ccol, cval, oa, ob, da, db, ld, acc);
+    if (d < ndet) ph_cross_dets<1>(d, ndet, cn, crow, ccol, cval, oa, ob, da, db, ld, acc);
   }
   acc = block_sum<256>(acc, red);
   if (tid == 0) out[(long)w * nch + chunk] = acc;
+}
+
+// Slices of a chunk (CH) and the pitch of its LDS rows (ld, 0: read in place) of k_ph_cross.  LDS: as many
+// slices as two workgroups a CU leave room for, 16 at most, at pitches that spread the rows over the
+// banks.  Time (128 walkers, 320 vectors, C configurations of both spins, D determinants): in LDS about
+// 0.26 C + (0.015 + 0.08 / CH) D us and more for CH <= 2, in place 0.095 C + 0.107 D, so LDS pays
+// from D / C of about 2 (CH = 9) to 4 (CH = 2) on.  Measured, LDS against in place: C = 227, D = 250 55
+// and 49 us; 455, 1000 137 and 149; 501, 2000 180 and 253; 504, 12000 410 and 1331; 1163, 2000 370
+// and 360; 1682, 4000 827 and 690; 1848, 16000 1495 and 2026; 4834, 16000 4031 and 2600.
+struct CrossShape {
+  int CH, ld;
+};
+CrossShape ph_cross_shape(long C, long D) {
+  int ld = (int)std::min<long>(17, 76L * 1024 / ((long)sizeof(z64) * C));
+  if (ld >= 8 && ld % 2 == 0) --ld;
+  const int CH = std::min(ld, 16);
+  if (D * (8 * CH - 9) > 14 * C * CH) return {CH, ld};
+  return {16, 0};
 }
 
 // energy_alg1 assembly per walker: reference terms times Ov, weighted excitation terms of both
@@ -1169,24 +1213,17 @@ void PhmsdTrial::energy(const z64* Pa, const z64* Pb, int W, z64* E, z64* Ov, lo
     else go(k_ph_energy_exc<6>);
     AFQ_LAUNCH_CHECK();
   }
-  // opposite-spin Coulomb term over Cholesky chunks of CH slices
+  // opposite-spin Coulomb term over chunks of Cholesky slices
   const int na = sp_[0].nconf, nb = sp_[1].nconf;
-  // (both spins' slices of a chunk in LDS, two workgroups a CU; read in place for larger
-  // expansions).  CH a power of two: rows of KE are read in whole 128-byte lines.  The LDS rows are
-  // one longer, or every determinant's j-th value would lie on two of the sixteen 16-byte bank
-  // groups.  Bound by the staging of KE; with the determinants eight at a time 256 walkers of 2000
-  // determinants take 416 us, one at a time and unpadded rows of 8 441 us.
-  const long fit = (76L * 1024) / ((long)sizeof(z64) * (na + nb));
-  const int use_lds = fit >= 2 ? 1 : 0;
-  int CH = 16;
-  while (use_lds && CH + 1 > fit) CH /= 2;
-  const int ncross = ceil_div(M, CH);
+  const CrossShape cs = ph_cross_shape(na + nb, ndet_);
+  const int ncross = ceil_div(M, cs.CH);
   z64* cross = scratch_as<z64>(ctx_, "ph_cross", (size_t)W * ncross);
-  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k_ph_cross),
+  auto k_cross = cs.ld ? k_ph_cross<true> : k_ph_cross<false>;
+  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k_cross),
                             hipFuncAttributeMaxDynamicSharedMemorySize, 76 * 1024);
-  hipLaunchKernelGGL(k_ph_cross, dim3(ncross, W), dim3(256),
-                     use_lds ? sizeof(z64) * (size_t)(na + nb) * (CH + 1) : 0, s, na, nb, M, CH,
-                     use_lds, ndet_, crow_, sp_[0].ccol, sp_[0].cval,
+  hipLaunchKernelGGL(k_cross, dim3(ncross, W), dim3(256),
+                     sizeof(z64) * (size_t)(na + nb) * cs.ld, s, na, nb, M, cs.CH, cs.ld, ndet_,
+                     crow_, sp_[0].ccol, sp_[0].cval,
                      scratch_as<z64>(ctx_, "ph_ovr0", (size_t)W * na),
                      scratch_as<z64>(ctx_, "ph_ovr1", (size_t)W * nb), KE[0], KE[1], cross);
   AFQ_LAUNCH_CHECK();

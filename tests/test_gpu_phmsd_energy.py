@@ -1,7 +1,9 @@
 """The particle-hole energy kernel at the edges of its work split, against the oracle, to the
 1e-10 bar of test_gpu_phmsd: slices in one, exactly full and one-over LDS runs, a single
-excitation, fewer and more electrons than the eight lanes that share a slice, every rank up to six,
-more configurations of one rank than threads, and a slice that leaves a CU to one workgroup.
+excitation, fewer and more electrons than the eight lanes that share a slice, ranks up to six, more
+configurations of one rank than threads, thousands of configurations with a number of vectors that
+is no multiple of the opposite-spin kernel's eight or sixteen, and a slice that leaves a CU to one
+workgroup.
 """
 import pytest
 
@@ -16,6 +18,8 @@ from test_gpu_phmsd import TOL, gpu, rel, rel_log, say, setup_case  # noqa: E402
     (dict(N=16, nel=5, M=32, ndet=30, ncore=0, nactive=9, max_rank=4, seed=33), 4),
     (dict(N=20, nel=9, M=33, ndet=50, ncore=2, nactive=12, max_rank=5, seed=34), 3),
     (dict(N=30, nel=12, M=17, ndet=900, ncore=2, nactive=20, max_rank=2, seed=35), 2),
+    (dict(N=16, nel=6, M=20, ndet=150, ncore=0, nactive=14, max_rank=6, seed=37), 2),
+    (dict(N=24, nel=8, M=26, ndet=6000, ncore=0, nactive=20, max_rank=2, seed=38), 2),
     (dict(N=66, nel=36, M=5, ndet=12, ncore=30, nactive=34, max_rank=3, seed=36), 2),
 ])
 def test_energy(gpu, kw, W):  # noqa: F811
