@@ -772,8 +772,11 @@ bool propagate_split(Context& c, const PropagateArgs& a) {
     else AFQ_PSP(2, 1);
 #undef AFQ_PSP
   };
-  tuned_on_copy(c, tune_key("prop_fused", sizeof(float), a.W, N, n, N), ncand, a.Phi,
-                (size_t)a.W * a.phi_bs, run);
+  // (a candidate means other work with another kind of P1 or number of 8-column groups)
+  tuned_on_copy(c,
+                tune_key("prop_fused", sizeof(float), a.W, N, n, N) + (p1c ? ":c" : ":r") +
+                    std::to_string(n8),
+                ncand, a.Phi, (size_t)a.W * a.phi_bs, run);
   return true;
 }
 

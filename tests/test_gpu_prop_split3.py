@@ -67,19 +67,25 @@ def test_against_fp64(gpu, N, n, W):
     assert np.all(np.abs(got - P1 @ S) <= 2 * c * (np.abs(P1) @ Sa))
 
 
-@pytest.mark.parametrize("N,n,W", [(40, 40, 3), (97, 23, 5), (200, 40, 4)])
+@pytest.mark.parametrize("N,n,W", [(40, 40, 3), (97, 23, 5), (200, 40, 4), (70, 64, 3)])
 def test_workgroups_per_walker_keep_the_bits(gpu, N, n, W):
     afq, ctx, torch = gpu
     print(f"case: split propagation, every candidate N={N} n={n} W={W}", flush=True)
     P1, V, Phi = inputs(N, n, W)
     ref = propagate(afq, ctx, P1, V, Phi)
-    for i in range(3):
+    # fewer and fewer of the n8 groups of 8 columns a workgroup, from five on, four candidates at most
+    n8 = -(-n // 8)
+    widths = sorted({-(-n8 // k) for k in range(-(-n8 // 5), n8 + 1)}, reverse=True)[:4]
+    for i in range(len(widths) + 1):
         afq.tune_force("prop_fused:f32", i)
         try:
-            got = propagate(afq, ctx, P1, V, Phi)
+            if i == len(widths):
+                with pytest.raises(afq.AfqError):
+                    propagate(afq, ctx, P1, V, Phi)
+            else:
+                assert np.array_equal(propagate(afq, ctx, P1, V, Phi), ref), i
         finally:
             afq.tune_force("prop_fused:f32", -1)
-        assert np.array_equal(got, ref), i
 
 
 @pytest.mark.parametrize("N,n", [(45, 11), (97, 24), (200, 40)])
@@ -186,3 +192,13 @@ def test_overflow(gpu):
     got = propagate(afq, ctx, np.ones((1, 1), np.complex128),
                     np.full((1, 1, 1), 3e38, np.complex64), np.full((1, 1, 1), 1.5 + 0j), 1)[0, 0, 0]
     assert np.isnan(got.real) and got.imag == np.inf
+
+
+def test_tuned_choices_are_not_shared_between_candidate_lists(gpu):
+    """48 and 64 columns have three and four candidates: each keeps a choice of its own."""
+    afq, ctx, torch = gpu
+    print("case: split propagation, tuning keys", flush=True)
+    for n in (48, 64):
+        propagate(afq, ctx, *inputs(190, n, 9))
+    lines = [x for x in afq.tuning_report().splitlines() if x.startswith("prop_fused:f32:16x256x64x")]
+    assert sorted(x.rsplit(" of ", 1)[1] for x in lines) == ["3", "4"]
