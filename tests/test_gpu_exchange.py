@@ -20,6 +20,7 @@ pytestmark = pytest.mark.gpu
 
 import oracle as orc  # noqa: E402
 from safire_amd.synthetic import make_problem, random_walkers  # noqa: E402
+from test_split_accuracy import PRODUCT, rel2  # noqa: E402
 
 BOUND = 2e-5
 
@@ -219,3 +220,27 @@ def test_walker_runs(gpu):
     every = _energies(afq, torch, ham, G, W, afq.AFQ_MIXED)
     last = _energies(afq, torch, ham, G[-201:].contiguous(), 201, afq.AFQ_MIXED)
     assert np.array_equal(every[-201:], last)
+
+
+# every tile size, N on and off the 32-wide groups, odd walkers and vectors
+@pytest.mark.parametrize("N,n,M,W", [(9, 1, 5, 3), (24, 8, 33, 7), (37, 13, 46, 5), (64, 24, 50, 6),
+                                     (97, 29, 31, 4), (200, 40, 64, 5)])
+def test_products_are_fp32(gpu, N, n, M, W):
+    """The Coulomb vectors tr T^m and the exchange energies, against 64 bits on the FP32 operands, in
+    the 2-norm that a lost partial product of the split exceeds (test_split_accuracy)."""
+    afq, torch = gpu
+    say(f"case: fused exchange accuracy N={N} n={n} M={M} W={W}")
+    p = make_problem(N, n, M, seed=79)
+    ctx = afq.Context(0)
+    ham = afq.HamiltonianOperations(ctx, p.h1, p.Likn, p.PsiT, n, precision=afq.AFQ_MIXED)
+    rng = np.random.default_rng(N)
+    G = rng.normal(size=(W, n, N)) + 1j * rng.normal(size=(W, n, N))
+    e = afq.empty((W, 3), torch.complex128)
+    k = afq.empty((W, M), torch.complex128)
+    ham.energy_spin(0, e, afq.device_tensor(G), k, precision=afq.AFQ_MIXED)
+    L = ham.tensors()[0].real.reshape(M, n, N).astype(np.float32).astype(np.float64)
+    T = np.einsum("wbk,mak->wmba", G.astype(np.complex64).astype(np.complex128), L)
+    K, X = np.trace(T, axis1=2, axis2=3), -np.einsum("wmba,wmab->w", T, T)
+    ek, ex = rel2(afq.host(k), K), rel2(afq.host(e)[:, 1], X)
+    say(f"  tr T {ek:.1e}, exchange {ex:.1e}")
+    assert ek <= PRODUCT and ex <= PRODUCT
