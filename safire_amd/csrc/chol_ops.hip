@@ -323,26 +323,24 @@ void CholeskyOps::vbias(const z64* G, int W, double dt, z64* v, Precision prec) 
     size_t goff = sp == 0 ? 0 : (size_t)nup_ * N_;
     size_t loff = sp == 0 ? 0 : (size_t)M_ * nup_ * N_;
     const long K = (long)ns * N_;
-    {
-      // A(w, (a,k)) = G[w][off + a][k]: rows of length nel*N, K = ns*N contiguous
-      Opnd<double, true, true> A{&(G + goff)->re, (long)nel_ * N_, 0};
-      EpiStore<double, double> e{v, M_, 0, a, 0, acc};
-      int ks = 0, kc = 0;
-      if (real_trial_ && crg_path() &&
-          crg::crg_supported<double>(G + goff, (long)nel_ * N_, W, Lnak_r_ + loff, K, M_))
-        crg::crg_split(W, M_, (int)K, 4, 3, ks, kc);
-      if (ks > 0 && crg::crg_fills(W, M_, 4, 3, ks)) {
-        // register-tiled, K cut into slices so that the 64 x 48 tiles fill the machine
-        z64* ws = ks > 1 ? scratch_as<z64>(ctx_, "crg_ws64", (size_t)ks * W * M_) : nullptr;
-        crg::launch_crgemm<double, 4, 3, false>(s, W, M_, (int)K, G + goff, (long)nel_ * N_,
-                                                Lnak_r_ + loff, crg::RowsPlain{K}, ks, kc, e, ws);
-      } else if (real_trial_) {
-        Opnd<double, false, true> B{Lnak_r_ + loff, K, 0};
-        gemm_large_splitk<double>(ctx_, "vbias_r", W, M_, (int)K, A, B, e, acc == 0);
-      } else {
-        Opnd<double, true, true> B{&(Lnak_ + loff)->re, K, 0};
-        gemm_large_splitk<double>(ctx_, "vbias_c", W, M_, (int)K, A, B, e, acc == 0);
-      }
+    // A(w, (a,k)) = G[w][off + a][k]: rows of length nel*N, K = ns*N contiguous
+    Opnd<double, true, true> A{&(G + goff)->re, (long)nel_ * N_, 0};
+    EpiStore<double, double> e{v, M_, 0, a, 0, acc};
+    int ks = 0, kc = 0;
+    if (real_trial_ && crg_path() &&
+        crg::crg_supported<double>(G + goff, (long)nel_ * N_, W, Lnak_r_ + loff, K, M_))
+      crg::crg_split(W, M_, (int)K, 4, 3, ks, kc);
+    if (ks > 0 && crg::crg_fills(W, M_, 4, 3, ks)) {
+      // register-tiled, K cut into slices so that the 64 x 48 tiles fill the machine
+      z64* ws = ks > 1 ? scratch_as<z64>(ctx_, "crg_ws64", (size_t)ks * W * M_) : nullptr;
+      crg::launch_crgemm<double, 4, 3, false>(s, W, M_, (int)K, G + goff, (long)nel_ * N_,
+                                              Lnak_r_ + loff, crg::RowsPlain{K}, ks, kc, e, ws);
+    } else if (real_trial_) {
+      Opnd<double, false, true> B{Lnak_r_ + loff, K, 0};
+      gemm_large_splitk<double>(ctx_, "vbias_r", W, M_, (int)K, A, B, e, acc == 0);
+    } else {
+      Opnd<double, true, true> B{&(Lnak_ + loff)->re, K, 0};
+      gemm_large_splitk<double>(ctx_, "vbias_c", W, M_, (int)K, A, B, e, acc == 0);
     }
   }
 }

@@ -865,68 +865,56 @@ bool propagate_fused(Context& c, const PropagateArgs& a, const T* P1, bool p1c, 
                    (reinterpret_cast<uintptr_t>(V) % 16) == 0;
   hipStream_t s = c.stream();
   const T* Vt = reinterpret_cast<const T*>(V);
-  // The V products by Gauss's three-multiplication method (three MFMAs per complex block
-  // instead of four): always in FP64; in FP32 only when AFQ_PROP_M3=1 (the four-product form
-  // keeps the FP32 rounding of the terms closer to the FP64 path's)
+  // The V products by Gauss's three-multiplication method (three MFMAs per complex block instead of
+  // four).  In FP32 one stripe per wave is reached with AFQ_PROP_M3=1, which asks for it, and at
+  // order 0, which has no V product (propagate_split takes the rest); two stripes per wave, beyond
+  // its N = 256, take four products unless asked, which keep the FP32 rounding of the terms closer to
+  // the FP64 path's.
   const char* m3e = std::getenv("AFQ_PROP_M3");
-  const bool m3 = sizeof(T) == 8 || (m3e && m3e[0] == '1');
+  const bool m3 = m3e && m3e[0] == '1';
   auto run = [&](int i, z64* Phi) {
     const int cb = cands[i].cb;
     const bool tail = cands[i].tail, split = cands[i].split;
-    constexpr int SPW2 = sizeof(T) == 4 ? 2 : 1;
-    if constexpr (sizeof(T) == 8) {
-      if (adj) {  // FP64 takes one stripe per wave and one column tile
-        if (p1c) launch_fused<T, true, 1, 1, true, true>(s, a, f, P1, vecP, Vt, vecV, Phi);
-        else launch_fused<T, false, 1, 1, true, true>(s, a, f, P1, vecP, Vt, vecV, Phi);
-        return;
-      }
-    }
-#define AFQ_PT(P1C, SPW, CB, TL)                                                         \
-  (m3 ? launch_fused<T, P1C, SPW, CB, false, true, TL>(s, a, f, P1, vecP, Vt, vecV, Phi) \
-      : launch_fused<T, P1C, SPW, CB, false, sizeof(T) == 8, TL>(s, a, f, P1, vecP, Vt, vecV, Phi))
-#define AFQ_PS(P1C, CB)                                                                          \
-  (m3 ? launch_fused<T, P1C, 1, CB, false, true, false, true>(s, a, f, P1, vecP, Vt, vecV, Phi) \
-      : launch_fused<T, P1C, 1, CB, false, sizeof(T) == 8, false, true>(s, a, f, P1, vecP, Vt,    \
-                                                                       vecV, Phi))
-    if (split) {
-      if constexpr (sizeof(T) == 4) {
-        if (p1c) {
-          if (cb == 1) AFQ_PS(true, 1);
-          else if (cb == 2) AFQ_PS(true, 2);
-          else AFQ_PS(true, 3);
-        } else {
-          if (cb == 1) AFQ_PS(false, 1);
-          else if (cb == 2) AFQ_PS(false, 2);
-          else AFQ_PS(false, 3);
-        }
+#define AFQ_PT(P1C, SPW, CB, CONJV, M3, TAIL, KT) \
+  launch_fused<T, P1C, SPW, CB, CONJV, M3, TAIL, KT>(s, a, f, P1, vecP, Vt, vecV, Phi)
+    if constexpr (sizeof(T) == 8) {  // one stripe per wave and one column tile
+      if (p1c) {
+        if (adj) AFQ_PT(true, 1, 1, true, true, false, false);
+        else if (split) AFQ_PT(true, 1, 1, false, true, false, true);
+        else AFQ_PT(true, 1, 1, false, true, false, false);
       } else {
-        if (p1c) AFQ_PS(true, 1);
-        else AFQ_PS(false, 1);
+        if (adj) AFQ_PT(false, 1, 1, true, true, false, false);
+        else if (split) AFQ_PT(false, 1, 1, false, true, false, true);
+        else AFQ_PT(false, 1, 1, false, true, false, false);
       }
-    } else if (f.spw == 1) {
-      if constexpr (sizeof(T) == 4) {
-        if (p1c) {
-          if (cb == 1) AFQ_PT(true, 1, 1, false);
-          else if (cb == 2) tail ? AFQ_PT(true, 1, 2, true) : AFQ_PT(true, 1, 2, false);
-          else tail ? AFQ_PT(true, 1, 3, true) : AFQ_PT(true, 1, 3, false);
-        } else {
-          if (cb == 1) AFQ_PT(false, 1, 1, false);
-          else if (cb == 2) tail ? AFQ_PT(false, 1, 2, true) : AFQ_PT(false, 1, 2, false);
-          else tail ? AFQ_PT(false, 1, 3, true) : AFQ_PT(false, 1, 3, false);
-        }
+    } else if (f.spw == 2) {
+      if (p1c) {
+        if (m3) AFQ_PT(true, 2, 1, false, true, false, false);
+        else AFQ_PT(true, 2, 1, false, false, false, false);
       } else {
-        if (p1c) AFQ_PT(true, 1, 1, false);
-        else AFQ_PT(false, 1, 1, false);
+        if (m3) AFQ_PT(false, 2, 1, false, true, false, false);
+        else AFQ_PT(false, 2, 1, false, false, false, false);
       }
     } else {
-      if (p1c) AFQ_PT(true, SPW2, 1, false);
-      else AFQ_PT(false, SPW2, 1, false);
+#define AFQ_PC(P1C)                                                     \
+  do {                                                                  \
+    if (cb == 1) AFQ_PT(P1C, 1, 1, false, true, false, false);          \
+    else if (cb == 2 && tail) AFQ_PT(P1C, 1, 2, false, true, true, false); \
+    else if (cb == 2) AFQ_PT(P1C, 1, 2, false, true, false, false);     \
+    else if (tail) AFQ_PT(P1C, 1, 3, false, true, true, false);         \
+    else AFQ_PT(P1C, 1, 3, false, true, false, false);                  \
+  } while (0)
+      if (p1c) AFQ_PC(true);
+      else AFQ_PC(false);
+#undef AFQ_PC
     }
 #undef AFQ_PT
-#undef AFQ_PS
   };
-  tuned_on_copy(c, tune_key(adj ? "prop_fused_adj" : "prop_fused", sizeof(T), W, N, n, N), ncand,
-                a.Phi, (size_t)W * a.phi_bs, run);
+  // (FP32 with one stripe per wave has candidates of its own, not propagate_split's)
+  const char* site = adj ? "prop_fused_adj"
+                     : sizeof(T) == 4 && f.spw == 1 ? "prop_taylor"
+                                                    : "prop_fused";
+  tuned_on_copy(c, tune_key(site, sizeof(T), W, N, n, N), ncand, a.Phi, (size_t)W * a.phi_bs, run);
   return true;
 }
 

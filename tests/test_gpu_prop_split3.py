@@ -69,6 +69,34 @@ def test_against_fp64(gpu, N, n, W):
     assert np.all(np.abs(got - P1 @ S) <= 2 * c * (np.abs(P1) @ Sa))
 
 
+# The FP32 kernel: beyond sixteen stripes, and below with the three-product form or without a V
+# product.  A sum of N terms takes N roundings, N u in the worst case and about the square root of it
+# (17 u) in the 2-norm, of each term falling by k!; three products lose up to another factor of four
+# (sums of two operands and of three results).
+@pytest.mark.parametrize("N,n,W,order,m3", [(257, 9, 2, 6, False), (300, 40, 2, 6, False),
+                                            (300, 17, 2, 6, True), (97, 23, 2, 6, True),
+                                            (200, 40, 2, 6, True), (50, 11, 2, 0, False),
+                                            (128, 40, 2, 0, False), (270, 20, 2, 0, False)])
+def test_fp32_kernel(gpu, monkeypatch, N, n, W, order, m3):
+    afq, ctx, torch = gpu
+    print(f"case: FP32 propagation N={N} n={n} W={W} order={order} m3={m3}", flush=True)
+    if m3:
+        monkeypatch.setenv("AFQ_PROP_M3", "1")
+    P1, V, Phi = inputs(N, n, W)
+    got = propagate(afq, ctx, P1, V, Phi, order)
+    T = P1 @ Phi
+    S = T.copy()
+    Ta = np.abs(P1) @ np.abs(Phi)
+    Sa = Ta.copy()
+    for k in range(1, order + 1):
+        T = (1j / k) * (V.astype(np.complex128) @ T)
+        Ta = (np.abs(V).astype(np.float64) @ Ta) / k
+        S, Sa = S + T, Sa + Ta
+    c = (order + 2) * (N + 4) * U
+    assert np.all(np.abs(got - P1 @ S) <= (8 if m3 else 2) * c * (np.abs(P1) @ Sa))
+    assert rel2(got, P1 @ S) <= (4 if m3 else 1) * 2 * PROPAGATION
+
+
 @pytest.mark.parametrize("N,n,W", [(40, 40, 3), (97, 23, 5), (200, 40, 4), (70, 64, 3)])
 def test_workgroups_per_walker_keep_the_bits(gpu, N, n, W):
     afq, ctx, torch = gpu
