@@ -534,17 +534,20 @@ __device__ __attribute__((noinline)) void redo_plain(Tile a, int tid, uint32_t* 
     for (int i = 0; i < WAVES; ++i) any = any || votes[i];
     return __ballot(any) != 0;
   };
-  // a column without a NaN
-  bool clean = false;
-  for (int c = tid; c < a.c1 - a.c0; c += TH) {
-    bool nan = false;
-    for (int k = 0; k < N; ++k) {
-      const z64 v = a.Pw[(long)k * a.n + a.c0 + c];
-      nan = nan || v.re != v.re || v.im != v.im;
+  // a column without a NaN (a dead walker's have one in the first row)
+  auto clean = [&](int rows) {
+    bool any = false;
+    for (int c = tid; c < a.c1 - a.c0; c += TH) {
+      bool nan = false;
+      for (int k = 0; k < rows; ++k) {
+        const z64 v = a.Pw[(long)k * a.n + a.c0 + c];
+        nan = nan || v.re != v.re || v.im != v.im;
+      }
+      any = any || !nan;
     }
-    clean = clean || !nan;
-  }
-  bool products = vote(clean);
+    return any;
+  };
+  bool products = vote(clean(1)) && vote(clean(N));
   if (products) {
     bool nan = false;
     for (int t = tid; t < 2 * N * N; t += TH) {

@@ -261,20 +261,23 @@ __device__ inline void redo_non_finite(f32x4 (&c)[RA][CB], __amdgpu_buffer_rsrc_
   bool need = false;
 #pragma unroll
   for (int i = 0; i < RA; ++i) {
-    bool nan = false;
-    for (int u = g0; u < g0 + gn; ++u) {
-      const bf16x8 p = load_block<0>(rA, oa[i] + (uint32_t)(u * (int)kBlock), l16);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) nan = nan || p[e] != p[e];
-    }
-    uint64_t rows = __ballot(nan);
-    rows |= rows >> 32;
-    rows |= rows >> 16;
+    uint32_t rows = 0;  // the lane's rows with such an accumulator
 #pragma unroll
     for (int j = 0; j < CB; ++j)
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        need = need || (!__builtin_isfinite(c[i][j][r]) && !(rows >> (4 * fk + r) & 1u));
+      for (int r = 0; r < 4; ++r) rows |= !__builtin_isfinite(c[i][j][r]) ? 1u << (4 * fk + r) : 0u;
+    // until each of them has shown a NaN: a dead walker's does in the first group
+    for (int u = g0; u < g0 + gn && __ballot(rows != 0) != 0; ++u) {  // uniform
+      const bf16x8 p = load_block<0>(rA, oa[i] + (uint32_t)(u * (int)kBlock), l16);
+      bool nan = false;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) nan = nan || p[e] != p[e];
+      uint64_t q = __ballot(nan);
+      q |= q >> 32;
+      q |= q >> 16;
+      rows &= ~(uint32_t)q;
+    }
+    need = need || rows != 0;
   }
   if (__ballot(need) == 0) return;  // uniform
 #pragma unroll
