@@ -5,7 +5,7 @@ Cholesky vectors, 1024 walkers, dt=0.005, 6-term Taylor propagator, QR every 5 s
 hamiltonian (safire_amd.synthetic, seed 1003) with Cholesky amplitude 0.1.  A step is one hybrid
 propagation of every walker (G, vbias, fields, vHS, P1 exp(iV) P1, overlap, weights) plus the
 growth estimator and Eshift relaxation, with the QR every fifth step, replayed from a HIP graph.
-`value` is the mixed precision path (FP32 MFMA contractions, FP64 G/LU/QR/weights); the FP64
+`value` is the mixed precision path (FP32 products on the bfloat16 cores, FP64 G/LU/QR/weights); the FP64
 path is timed beside it.  At the generator's default amplitude 0.5 the walkers' weights all
 reach zero within about four steps (the FP64 oracle shows the same) and the matrices overflow,
 so the timed steps would run on dead walkers and the mixed-vs-FP64 condition cannot be met;
@@ -34,7 +34,12 @@ RECIPE_AMPLITUDE = 0.5   # the generator's default
 # "mixed": an FP32 product is six bfloat16 products on the matrix cores (dense peak 2.5 PFLOP/s)
 PEAK = {"mixed": 2.5e15 / 6, "fp64": 78.6e12}
 HBM_PEAK = 8.0e12
-# bytes of one mixed vHS launch: X and the symmetric pairs of L as three bfloat16 pieces, V as c64
+# HBM bytes of one mixed vHS launch (k_split3_gemm over the symmetric pairs) at this workload:
+# FETCH_SIZE x 2 + WRITE_SIZE x 1 in KiB (the factors that make a 1 GiB copy read and write
+# 1 GiB), rocprofv3 --pmc of `bench.py --only step`
+# (profiles/step_N200_n40_M1600_W1024_pmc.md).  Algorithmic: X and the symmetric pairs of L as three
+# bfloat16 pieces, V as c64.
+VHS_TRAFFIC_BYTES = (914318 * 2 + 507203) * 1024
 VHS_ALGORITHMIC_BYTES = W * M * 12 + (N * (N + 1) // 2) * M * 6 + W * N * N * 8
 
 
@@ -755,7 +760,9 @@ def main():
                      "vhs_ms_in_step_graph_events": out["mixed"]["vhs"] * 1e3,
                      "achieved_in_step_graph_events": vhs_flops / out["mixed"]["vhs"] / 1e12,
                      "unit": "TFLOP/s", "frac": achieved / PEAK["mixed"],
-                     "algorithmic_bytes": VHS_ALGORITHMIC_BYTES},
+                     "algorithmic_bytes": VHS_ALGORITHMIC_BYTES,
+                     "traffic": VHS_TRAFFIC_BYTES,
+                     "traffic_over_algorithmic": VHS_TRAFFIC_BYTES / VHS_ALGORITHMIC_BYTES},
         # the whole step: the FLOP the kernels issue (flops_per_walker_step) per second over the
         # MFMA peak of the contraction precision; *_all_complex: the count with every MAC
         # complex and vHS over all N^2 entries

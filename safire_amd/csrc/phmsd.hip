@@ -520,7 +520,8 @@ struct PhRanks {
 // Bound by FP64 vector products (45 complex ones for an excitation of rank 3 and a slice) and by the
 // reading of T.  256 walkers, 321 slices, 15 x 10 active orbitals, 2000 determinants, both spins: a
 // kernel per rank with the sum over l in it and one for jr and tz 2.6 ms, this kernel 0.80 ms.
-// RMAX: the largest rank (4 keeps two workgroups a CU within the register file).
+// RMAX: the largest rank (4 keeps two workgroups a CU within the register file, with 16 bytes a lane
+// spilled; 6 spills 116).
 template <int RMAX>
 __global__ void __launch_bounds__(256, RMAX <= 4 ? 2 : 1)
     k_ph_energy_exc(int nel, int nact, int nconf, int M, int NS, int NC, PhRanks ranks,

@@ -36,12 +36,14 @@
 // FP32 range: the tile enters scaled by 2^-e, e the binary exponent of its largest entry, and
 // leaves scaled back by 2^e.
 //
-// Bound by the matrix cores and by V, which is read from memory once per term (the V of the
-// resident walkers does not fit the L2s).  Against the same recurrence on FP32 MFMAs (six terms;
-// errors against 64 bits 0.3 to 0.6 of its): N = 200, n = 40, 1024 walkers 1020 -> 659 us, 128 walkers
-// 189 -> 113 us, N = 97, n = 23, 301 walkers 97 -> 75 us; with a complex P1 N = 24, n = 5, 64 walkers
-// 13.4 -> 11.3 us, N = 160, n = 40, 256 walkers 192 -> 179 us (its pieces spill).  So every size and
-// both kinds of P1 that fit take this kernel.
+// Bound by the matrix cores and by V, which is read from memory once per term (the V of the resident
+// walkers does not fit the L2s): the cores are busy 45 % of the time at N = 200.  Against the same
+// recurrence on FP32 MFMAs (six terms; errors against 64 bits 0.3 to 0.6 of its): N = 200, n = 40,
+// 1024 walkers 1020 -> 639 us, 128 walkers 189 -> 113 us, N = 97, n = 23, 301 walkers 97 -> 75 us;
+// with a complex P1 N = 24, n = 5, 64 walkers 13.4 -> 11.3 us, N = 160, n = 40, 256 walkers 192 -> 179
+// us.  Above 16 columns and N = 64 the registers do not suffice: 32 to 144 bytes a lane are spilled,
+// outside the k loops, and with a complex P1 up to 720.  So every size and both kinds of P1 that fit take
+// this kernel.
 #include <cstdlib>
 #include <type_traits>
 

@@ -1,15 +1,17 @@
 // FP32 products on the bfloat16 matrix cores: every FP32 operand is split into three bfloat16
-// numbers, x = x0 + x1 + x2, exactly (24 significand bits in three pieces of 8, rounded to nearest),
-// and a product keeps the six partial products above 2^-24 of it,
+// numbers, x = x0 + x1 + x2, exactly (24 significand bits in three pieces of 8, rounded to nearest;
+// the method of Henry, Tang and Heinecke, "Leveraging the bfloat16 artificial intelligence datatype
+// for higher-precision computations", ARITH 2019), and a product keeps the six partial products above
+// 2^-24 of it,
 //
 //   a b  ~  a0 b2 + a2 b0 + a0 b1 + a0 b0 + a1 b0 + a1 b1        (left out: a1 b2, a2 b1, a2 b2)
 //
 // each exact in FP32 and accumulated in FP32 by v_mfma_f32_16x16x32_bf16.
 //
 // Why: the FP32 MFMA rate is 1/16 of the bfloat16 rate, so six bfloat16 MFMAs cost 6/16 of the
-// FP32 MFMAs they replace.  The error is below that of v_mfma_f32_16x16x4f32: the six MFMAs of 32 k
-// values are summed from zero and added to the accumulator once, where the FP32 MFMA rounds the
-// accumulator at every step.  Measured against FP64 over 1600 terms falling as exp(-k/20),
+// FP32 MFMAs they replace.  The error is below that of v_mfma_f32_16x16x4f32: k_split3_gemm sums the six
+// MFMAs of 32 k values from zero and adds them to the accumulator once, where the FP32 MFMA rounds
+// the accumulator at every step.  Measured against FP64 over 1600 terms falling as exp(-k/20),
 // smallest first (2-norm of the error over that of the result): 5.0e-8, FP32 MFMA 8.1e-8.
 //
 // Packed operands.  The split operands are laid out so that one MFMA operand of a wavefront is
@@ -113,8 +115,9 @@ struct RowsItems {
 
 // One wavefront per (16-row block, k group) of a complex operand X [rows][ld].  Blocks of nb rows
 // form a tile: block i of tile t holds its real parts at block row (2 t) nb + i of `out` and its
-// imaginary parts at (2 t + 1) nb + i.  Reads 8 (TIn float) or 16 bytes a value and writes 12:
-// bound by memory.
+// imaginary parts at (2 t + 1) nb + i.  Reads 8 (TIn float) or 16 bytes a value and writes 12: 4.3 TB/s
+// from FP32 (G of 1024 walkers, N = 200, n = 40: 38 us), 1.9 TB/s from FP64, whose loads touch twice
+// the lines; a copy reaches 5.
 template <typename TIn, class ROWS>
 __global__ void __launch_bounds__(256)
     k_pack_cplx(long blocks, int K0, int KG0, int K, int KG, const cplx<TIn>* __restrict__ X,
@@ -322,9 +325,10 @@ __device__ inline void redo_non_finite(f32x4 (&c)[RA][CB], __amdgpu_buffer_rsrc_
 // smallest first).  Split-K slices pass ks to the epilogue: ks0 slices of kchunk groups of the first
 // KG0 groups, then those of the others (the two spins of vbias, whose sums stay apart).
 //
-// Bound by the matrix cores and their operand feed through L2.  Measured (1024 x 20100 outputs
-// over 1600): 0.60 ms = 220 TFLOP/s of FP32 products, 0.57 of what six back-to-back MFMAs reach on
-// this card (2.33 PFLOP/s / 6); with the FP32 MFMA 1.18 ms.  Eight wavefronts per workgroup or a
+// Bound by the operand feed through L2: the matrix cores are busy half of the time.  Measured in a
+// walker step (1024 x 20100 outputs over 1600): 0.75 ms = 177 TFLOP/s of FP32 products, 0.46 of what six
+// back-to-back MFMAs reach on this card (2.33 PFLOP/s / 6); with the FP32 MFMA 1.13 ms.  Repeated on
+// fields of full amplitude it takes 0.77 to 0.93 ms.  Eight wavefronts per workgroup or a
 // barrier per k group (more reuse in L1) measured 2-18 % slower.
 template <int RB, int CB, bool REVK, class EPI>
 __global__ void __launch_bounds__(256, 2)

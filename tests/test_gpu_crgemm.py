@@ -1,11 +1,13 @@
-"""The register-tiled FP32 complex x real product (crgemm.hpp) behind the mixed-precision vHS.
+"""The products that AFQ_CRGEMM=0 switches off: the split bfloat16 vHS of the mixed precision
+(split3.hpp) and the register-tiled FP64 vHS and vbias (crgemm.hpp).
 
 Checks, through the C ABI: against the FP64 oracle's vHS within the FP32 bound (the inputs
 rounded to FP32 and an FP32 sum over M terms: relative error below 1e-5 of the largest entry,
-with the largest per-walker error stated); against the LDS-staged GEMM engine it replaces
-(AFQ_CRGEMM=0) within the same bound; bit-for-bit repeatable; exactly symmetric V; at shapes
-whose walkers, pairs and Cholesky vectors fall off the 64 x 112 x 16 tiling (clamped rows,
-invalid pairs and a ragged k group, taken first with the reversed order).
+with the largest per-walker error stated); against the LDS-staged GEMM engine they replace
+(AFQ_CRGEMM=0) within the same bound; bit-for-bit repeatable; exactly symmetric V; whole mixed
+steps; at shapes whose walkers, pairs and Cholesky vectors fall off the 32 x 96 x 32 (mixed) and
+64 x 48 x 16 (FP64) tilings.  tests/test_gpu_split3.py goes through the edges of the split
+product one by one.
 """
 import os
 import sys
@@ -51,12 +53,12 @@ def _vhs(afq, torch, ham, X, N, crg):
             os.environ["AFQ_CRGEMM"] = old
 
 
-# M % 4 != 0 (the last case) is outside the kernel's alignment: both runs take the GEMM engine
+# (the last case's M is no multiple of the 16-byte words of the FP64 kernel; the split has no such limit)
 @pytest.mark.parametrize("N,M,W", [(200, 1600, 96), (21, 40, 37), (64, 332, 130), (8, 20, 5),
                                    (10, 33, 7)])
 def test_crgemm_vhs(gpu, N, M, W):
     afq, ctx, torch = gpu
-    say(f"case: register-tiled vHS N={N} M={M} W={W}")
+    say(f"case: split vHS N={N} M={M} W={W}")
     p = make_problem(N, 4, M, 13)
     ham = afq.HamiltonianOperations(ctx, p.h1, p.Likn, p.PsiT, 4, precision=afq.AFQ_MIXED)
     rng = np.random.default_rng(5)

@@ -11,10 +11,10 @@ Bounds asserted:
   exceeds 0.1 mHa, so that bar is out of reach for any FP32 propagation there;
 * at both amplitudes every FP32 stage, and the mixed step, stays within 100 times the floor
   (maximum over walkers of |dE| / |E|): an FP32 contraction over K terms carries ~sqrt(K) u
-  relative error, sqrt(1600) = 40 for vHS, i.e. ~80 times the floor's u / 2 (measured: 20-60
-  times at amplitude 0.5, 5-35 times at 0.1);
+  relative error, sqrt(1600) = 40 for vHS, i.e. ~80 times the floor's u / 2 (measured: 6-57
+  times at amplitude 0.5, 3-27 times at 0.1);
 * at Cholesky amplitude 0.1 (local energies of ~600 Ha; the benchmark's workload) the mixed
-  step meets 0.1 mHa per walker (measured 9.3e-5 Ha at most over 128 walkers).
+  step meets 0.1 mHa per walker (measured 7.4e-5 Ha at most over 128 walkers).
 """
 import os
 import sys
