@@ -259,3 +259,67 @@ def test_two_spins_take_the_launches_of_one(gpu, N, n, nd, M, W):
                                 ctypes.byref(nodes)) == 0
     print("  nodes", nodes.value, flush=True)
     assert 2 <= nodes.value <= 3
+
+
+def test_fields_past_2_gib(gpu):
+    """Packed fields of more than 2 GiB (unsigned 32-bit offsets): the last walkers' V."""
+    afq, ctx, torch = gpu
+    N, M, W = 8, 1024, 180_000
+    print(f"case: split vHS, fields past 2 GiB N={N} M={M} W={W}", flush=True)
+    p = make_problem(N, 1, M, 3)
+    ham = afq.HamiltonianOperations(afq.Context(0), p.h1, p.Likn, p.PsiT, 1,
+                                    precision=afq.AFQ_MIXED)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    X = torch.randn(W, M, generator=g, dtype=torch.complex64, device="cuda")
+    V = afq.empty((W, N, N), torch.complex64)
+    ham.vHS(X, V, 1.0)
+    L = f32(p.Likn).reshape(N * N, M).astype(np.float64)
+    for rows in (slice(0, 40), slice(W - 40, W)):
+        ref = afq.host(X[rows]).astype(np.complex128) @ L.T
+        assert rel2(afq.host(V[rows]).reshape(40, -1), ref) <= PRODUCT
+
+
+def test_walkers_in_runs(gpu):
+    """A density matrix whose packed form passes 4 GiB is taken in runs of walkers."""
+    afq, ctx, torch = gpu
+    N, n, M, W = 64, 32, 5, 180_000
+    print(f"case: split vbias, walker runs N={N} n={n} M={M} W={W}", flush=True)
+    p = make_problem(N, n, M, 3)
+    ham = afq.HamiltonianOperations(afq.Context(0), p.h1, p.Likn, p.PsiT, n,
+                                    precision=afq.AFQ_MIXED)
+    g = torch.Generator(device="cuda").manual_seed(6)
+    G = torch.randn(W, n, N, generator=g, dtype=torch.complex128, device="cuda")
+    v = afq.empty((W, M), torch.complex128)
+    ham.vbias(G, v, 1.0)
+    L = f32(ham.tensors()[0].real.reshape(M, -1)).astype(np.float64)
+    for w0 in (0, 100_000, 170_000, W - 40):
+        ref = 2.0 * f32(afq.host(G[w0:w0 + 40]).reshape(40, -1)).astype(np.complex128) @ L.T
+        assert rel2(afq.host(v[w0:w0 + 40]), ref) <= PRODUCT
+
+
+def test_vectors_in_runs(gpu):
+    """Two spins' half-rotated rows of more than 4 GiB packed (each below it) are taken in runs of
+    vectors."""
+    afq, ctx, torch = gpu
+    N = n = 33
+    M, W = 350_000, 3
+    print(f"case: split vbias, vector runs N={N} n={n}+{n} M={M} W={W}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(9)
+    L = torch.randn(N, N, M, generator=g, dtype=torch.float64, device="cuda") / N
+    L = 0.5 * (L + L.transpose(0, 1))
+    rng = np.random.default_rng(9)
+    h1 = rng.normal(size=(N, N))
+    P = np.linalg.qr(rng.normal(size=(N, N)))[0]
+    ham = afq.HamiltonianOperations(afq.Context(0), 0.5 * (h1 + h1.T), L.cpu().numpy(),
+                                    np.concatenate([P, P]).astype(np.complex128), n, n,
+                                    walker_type=afq.AFQ_COLLINEAR, precision=afq.AFQ_MIXED)
+    G = afq.device_tensor(rng.normal(size=(W, 2 * n, N)) + 1j * rng.normal(size=(W, 2 * n, N)))
+    v = afq.empty((W, M), torch.complex128)
+    ham.vbias(G, v, 1.0)
+    # sum over a, k of G[a][k] sum_i P[a][i] L[i][k][m], both spins with the same P
+    F = torch.einsum("ai,wak->wik", afq.device_tensor(P).to(torch.complex128), G[:, :n] + G[:, n:])
+    F, L = F.reshape(W, -1), L.reshape(N * N, M)
+    ref = torch.complex(F.real.contiguous() @ L, F.imag.contiguous() @ L)
+    # (two more roundings to FP32, of G and of the half-rotated rows, are in the result)
+    for m in (slice(0, 1000), slice(M // 2, M // 2 + 1000), slice(M - 1000, M)):
+        assert rel2(afq.host(v[:, m]), afq.host(ref[:, m])) <= PRODUCT + 2 * U
